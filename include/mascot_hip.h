@@ -373,8 +373,8 @@ int mf_matrix_reconst_triplet(mf_node* R, const uint32_t* user2sorted_idx, const
 /* Seeded replacement for srand(time(0)); std::random_shuffle(R, R+n) (mf_methods.cu:38-39): out = in
  * permuted by ascending 64-bit key(seed, i).  Convenience form: allocates its workspace, frees it, synchronises. */
 int mf_shuffle_ratings(const mf_node* in, mf_node* out, uint32_t n, uint64_t seed, void* stream);
-/* The same with a caller-owned workspace (256-byte aligned, mf_shuffle_ratings_workspace_bytes(n) bytes: keys, ids,
- * the permutation and rocPRIM's temporary storage): asynchronous, allocates nothing, synchronises nothing. */
+/* The same with a caller-owned workspace (256-byte aligned, mf_shuffle_ratings_workspace_bytes(n) bytes: ratings and
+ * their positions after each of up to two partition passes, and the passes' counts): asynchronous, allocates nothing, synchronises nothing. */
 size_t mf_shuffle_ratings_workspace_bytes(uint32_t n);
 int mf_shuffle_ratings_ws(const mf_node* in, mf_node* out, uint32_t n, uint64_t seed, void* workspace, size_t workspace_bytes, void* stream);
 

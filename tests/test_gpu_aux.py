@@ -120,6 +120,56 @@ def test_histogram_sort_reindex(orc):
     assert np.array_equal(from_dev(dR, np.uint8), want.view(np.uint8).reshape(-1))
 
 
+@pytest.mark.parametrize("n", [1, 2, 63, 3072, 3073, 4097, 6145, 393217, 786432, 786433, 1572865, 3000001])
+def test_shuffle_sizes(orc, n):
+    """No partition pass (up to 3072 ratings), one (up to 256 buckets of 3072) and two, at the sizes where the number of
+    buckets changes and with tiles and chunks that end early; the permutation is unique, so it has to be the checker's."""
+    import torch
+    h = mfutil.hip()
+    R = np.zeros(n, mfutil.NODE)
+    R["r"], R["u"], R["i"] = np.arange(n) % 11, np.arange(n), np.arange(n)[::-1]
+    dR, dOut = to_dev(R), torch.full((n * 12,), 0xee, dtype=torch.uint8, device="cuda")
+    need = h.mf_shuffle_ratings_workspace_bytes(n)
+    ws = torch.full((need,), 0xa5, dtype=torch.uint8, device="cuda")
+    for seed in (5, 6):
+        h.mf_shuffle_ratings_ws(dR.data_ptr(), dOut.data_ptr(), n, seed, ws.data_ptr(), need, mfutil.stream_ptr())
+        torch.cuda.synchronize()
+        assert np.array_equal(from_dev(dOut, mfutil.NODE).view(np.uint8), orc.shuffle(seed, R).view(np.uint8))
+
+
+def test_shuffle_beyond_the_large_tiles():
+    """From 2^16 buckets of 3072 ratings on a pass has more than 8 bits and takes smaller tiles; against torch's sort of the keys."""
+    import torch
+    h, n, seed = mfutil.hip(), (3072 << 16) + 77, 9
+    R = torch.empty((n, 3), dtype=torch.int32, device="cuda")
+    for word in range(3):
+        R[:, word] = torch.arange(n, dtype=torch.int32, device="cuda") + word
+    out = torch.zeros_like(R)
+    need = h.mf_shuffle_ratings_workspace_bytes(n)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    h.mf_shuffle_ratings_ws(R.data_ptr(), out.data_ptr(), n, seed, ws.data_ptr(), need, mfutil.stream_ptr())
+    del ws
+
+    def signed(x):
+        x &= (1 << 64) - 1
+        return x - (1 << 64) if x >> 63 else x
+
+    def shifted(x, by):           # logical shift of 64-bit words held as signed ones
+        return (x >> by) & ((1 << (64 - by)) - 1)
+
+    def mix64(x):
+        x = x + signed(0x9E3779B97F4A7C15)
+        x = (x ^ shifted(x, 30)) * signed(0xBF58476D1CE4E5B9)
+        x = (x ^ shifted(x, 27)) * signed(0x94D049BB133111EB)
+        return x ^ shifted(x, 31)
+    base = mix64(torch.tensor([signed(seed ^ 0x53485546464C4521)], dtype=torch.int64, device="cuda"))
+    key = mix64(base ^ torch.arange(n, dtype=torch.int64, device="cuda")) ^ signed(1 << 63)      # unsigned order
+    order = torch.argsort(key).to(torch.int32)
+    del key
+    for word in range(3):
+        assert torch.equal(out[:, word], order + word)
+
+
 def test_shuffle_is_the_checkers_permutation(orc):
     import torch
     h = mfutil.hip()
