@@ -117,56 +117,152 @@ __global__ __launch_bounds__(kWave) void group_error_kernel(float* __restrict__ 
     if (lane == 0) error_out[g] = (acc / nacc) / initial[g];
 }
 
-// ---- test RMSE (rmse.h:26-189): wave reduction of each dot, per-wave double accumulation, LDS
-// reduction across the workgroup, one double atomic per workgroup ----------------------------------
-__device__ __forceinline__ void block_sum_to_global(double acc, double* out)
+// ---- test RMSE (rmse.h:26-189) ------------------------------------------------------------------------
+// A rating's rows are read by one row of 16 lanes, 16 bytes of a binary16 row per lane at k = 128: a wavefront has four
+// ratings per load and reduces four dots with four cross-lane adds.  Lane row w of a wavefront takes ratings 16 w .. 16 w + 15
+// of the wavefront's 64, four at a time, so that 16 loads are in flight; a rating's values come from the lane that holds it by
+// DPP broadcast within the row.
+// What bounds it is the row reads, which mostly hit in L2 (test sets are sorted by user).  With one rating per wavefront
+// step (one row per load, six cross-lane adds, loads waited for one rating at a time) 1.4M ratings of
+// a model of 480k x 17.8k rows at k = 128, a twentieth of the groups binary32, took 261 us; this takes 70, 10 TB/s of row reads.
+constexpr int kRmseBlock = 1024;
+constexpr uint32_t kRmseWaves = kRmseBlock / kWave;
+// One double atomic per workgroup, all on one address: two workgroups per compute unit at most.
+constexpr uint32_t kRmseGrid = 512;
+static inline uint32_t rmse_grid(uint32_t test_n)
 {
-    __shared__ double part[kWavesPerBlock];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) part[w] = acc;
+    const uint32_t blocks = (uint32_t)(((uint64_t)test_n + kRmseBlock - 1) / kRmseBlock);
+    return blocks < kRmseGrid ? blocks : kRmseGrid;
+}
+// Value of lane N of the same row of 16 lanes.
+template <int N, class T> __device__ __forceinline__ T row_bcast(T x)
+{
+    return from_bits<T>((uint32_t)__builtin_amdgcn_mov_dpp((int)bits(x), 0x150 + N, 0xf, 0xf, true));
+}
+template <int N> __device__ __forceinline__ uint64_t row_bcast64(uint64_t x)
+{
+    return (uint64_t)row_bcast<N>((uint32_t)x) | ((uint64_t)row_bcast<N>((uint32_t)(x >> 32)) << 32);
+}
+template <int N> __device__ __forceinline__ uint64_t row_ror64(uint64_t x)
+{
+    return (uint64_t)row_ror<N>((uint32_t)x) | ((uint64_t)row_ror<N>((uint32_t)(x >> 32)) << 32);
+}
+// K / 16 elements of a row as one lane reads them: K / 8 bytes of a binary16 row, or twice as many of a binary32 row in two
+// parts.  Rows are aligned to their elements only.
+template <int K> struct RowPart {
+    static constexpr int kWords = K / 32;
+    typedef uint32_t Words __attribute__((ext_vector_type(kWords)));
+    typedef Words Words2 __attribute__((aligned(2)));
+    Words lo, hi;
+    __device__ __forceinline__ void load_lo(uint64_t at) { lo = *(const MF_GLOBAL Words2*)at; }
+    __device__ __forceinline__ void load_hi(uint64_t at) { hi = *(const MF_GLOBAL Words2*)(at + sizeof(Words)); }
+    // element 2 w + b
+    __device__ __forceinline__ float half_at(int w, int b) const { const half2_t h = from_bits<half2_t>(lo[w]); return b ? (float)h.y : (float)h.x; }
+    __device__ __forceinline__ float single_at(int w, int b) const
+    {
+        const int e = 2 * w + b;
+        return from_bits<float>(e < kWords ? lo[e < kWords ? e : 0] : hi[e < kWords ? 0 : e - kWords]);
+    }
+};
+// One wavefront's rating per lane; flags: bit 0/1 the P/Q row is binary32, bit 2 there is no rating (or its id is in no group).
+struct TestRating { float r; uint64_t p, q; uint32_t flags; };
+// Adds the squared errors of the ratings in lanes 0 .. 3 of each lane row to acc (the same value in its 16 lanes).
+template <int K, bool SINGLE> __device__ __forceinline__ void rmse_four(const TestRating& my, uint32_t lane16, double& acc)
+{
+    RowPart<K> a[4], b[4];
+    uint64_t pa[4], qa[4]; uint32_t f[4]; float r[4];
+    auto fetch = [&](auto D) {
+        constexpr int d = decltype(D)::value;
+        f[d] = SINGLE ? row_bcast<d>(my.flags) | 3u : row_bcast<d>(my.flags);
+        r[d] = row_bcast<d>(my.r);
+        pa[d] = row_bcast64<d>(my.p) + (uint64_t)(lane16 * (K / 8) << (f[d] & 1u));
+        qa[d] = row_bcast64<d>(my.q) + (uint64_t)(lane16 * (K / 8) << ((f[d] >> 1) & 1u));
+        a[d].load_lo(pa[d]); b[d].load_lo(qa[d]);
+        if constexpr (SINGLE) { a[d].load_hi(pa[d]); b[d].load_hi(qa[d]); }
+    };
+    fetch(std::integral_constant<int, 0>()); fetch(std::integral_constant<int, 1>());
+    fetch(std::integral_constant<int, 2>()); fetch(std::integral_constant<int, 3>());
+    const bool any = SINGLE || __ballot(((f[0] | f[1] | f[2] | f[3]) & 3u) != 0u) != 0ull;
+    if (!SINGLE && any) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            if (f[d] & 1u) a[d].load_hi(pa[d]); else a[d].hi = a[d].lo;
+            if (f[d] & 2u) b[d].load_hi(qa[d]); else b[d].hi = b[d].lo;
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        float dot = 0.f;
+        if (any) {
+#pragma unroll
+            for (int w = 0; w < RowPart<K>::kWords; ++w)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    dot = __builtin_fmaf(SINGLE || (f[d] & 1u) ? a[d].single_at(w, e) : a[d].half_at(w, e),
+                                         SINGLE || (f[d] & 2u) ? b[d].single_at(w, e) : b[d].half_at(w, e), dot);
+        } else {
+#pragma unroll
+            for (int w = 0; w < RowPart<K>::kWords; ++w)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) dot = __builtin_fmaf(a[d].half_at(w, e), b[d].half_at(w, e), dot);
+        }
+        dot = reduce_row16(dot, OpAdd());
+        const double err = f[d] & 4u ? 0.0 : (double)(r[d] - dot);
+        acc += err * err;
+    }
+}
+// All ratings of a wavefront.  A lane without a rating reads the rows of one that has, and adds nothing.
+template <int K, bool SINGLE> __device__ __forceinline__ void rmse_wave(TestRating my, double& acc)
+{
+    const uint64_t valid = __ballot(!(my.flags & 4u));
+    if (!valid) return;
+    const int some = __builtin_ctzll(valid);
+    const uint64_t p = bcast(my.p, some), q = bcast(my.q, some); const uint32_t f = bcast(my.flags, some);
+    if (my.flags & 4u) { my.p = p; my.q = q; my.flags = f | 4u; }
+    const uint32_t lane16 = threadIdx.x & 15u;
+    // not unrolled: four batches' loads in flight at once would not fit the registers of 16 wavefronts per compute unit
+#pragma unroll 1
+    for (int batch = 0; batch < 4; ++batch) {
+        rmse_four<K, SINGLE>(my, lane16, acc);
+        my.r = row_ror<4>(my.r); my.flags = row_ror<4>(my.flags);
+        my.p = row_ror64<4>(my.p); my.q = row_ror64<4>(my.q);
+    }
+}
+__device__ __forceinline__ void rmse_block_sum(double acc, double* out)
+{
+    __shared__ double part[kRmseWaves * 4];
+    if ((threadIdx.x & 15u) == 0u) part[threadIdx.x >> 4] = acc;
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0;
-        for (int i = 0; i < kWavesPerBlock; ++i) s += part[i];
+        for (uint32_t i = 0; i < kRmseWaves * 4; ++i) s += part[i];
         atomicAdd(out, s);
     }
 }
 
 template <int K>
-__global__ __launch_bounds__(kBlock) void rmse_dense_kernel(const mf_node* __restrict__ test, uint32_t test_n, const float* __restrict__ P,
-                                                           const float* __restrict__ Q, double* sum_sq)
+__global__ __launch_bounds__(kRmseBlock) void rmse_dense_kernel(const mf_node* __restrict__ test, uint32_t test_n, const float* __restrict__ P,
+                                                               const float* __restrict__ Q, double* sum_sq)
 {
-    constexpr int E = K / 64;
-    const int lane = threadIdx.x & 63;
-    const uint32_t waves = gridDim.x * kWavesPerBlock;
-    const uint32_t wid = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
     double acc = 0;
-    for (uint64_t base = (uint64_t)wid * kWave; base < test_n; base += (uint64_t)waves * kWave) {
-        const uint64_t left = test_n - base;
-        const int n = left < (uint64_t)kWave ? (int)left : kWave;
-        Rating my = {0.f, 0u, 0u};
-        if (lane < n) my = load_rating(test, (uint32_t)(base + lane));
-        for (int j = 0; j < n; ++j) {
-            const float r = bcast(my.r, j);
-            const float* pp = P + (size_t)bcast(my.u, j) * K + lane;
-            const float* qq = Q + (size_t)bcast(my.v, j) * K + lane;
-            float d = pp[0] * qq[0];
-            if constexpr (E == 2) d = d + pp[64] * qq[64];
-            d = reduce_wave(d, OpAdd());
-            const double err = (double)(r - d);
-            acc += err * err;
+    for (uint64_t base = ((uint64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x) * kWave; base < test_n; base += (uint64_t)gridDim.x * kRmseBlock) {
+        TestRating my = {0.f, 0, 0, 7u};
+        if (base + lane < test_n) {
+            const Rating x = load_rating(test, (uint32_t)(base + lane));
+            my = {x.r, reinterpret_cast<uint64_t>(P) + (uint64_t)x.u * (K * 4u), reinterpret_cast<uint64_t>(Q) + (uint64_t)x.v * (K * 4u), 3u};
         }
+        rmse_wave<K, true>(my, acc);
     }
-    block_sum_to_global(acc, sum_sq);
+    rmse_block_sum(acc, sum_sq);
 }
 
 template <int K>
-__global__ __launch_bounds__(kBlock) void rmse_grouped_kernel(const mf_node* __restrict__ test, uint32_t test_n, void* const* __restrict__ p, void* const* __restrict__ q,
-                                                             const uint32_t* __restrict__ user_end, const uint32_t* __restrict__ item_end,
-                                                             const uint8_t* __restrict__ user_prec, const uint8_t* __restrict__ item_prec,
-                                                             uint32_t user_groups, uint32_t item_groups, double* sum_sq)
+__global__ __launch_bounds__(kRmseBlock) void rmse_grouped_kernel(const mf_node* __restrict__ test, uint32_t test_n, void* const* __restrict__ p, void* const* __restrict__ q,
+                                                                 const uint32_t* __restrict__ user_end, const uint32_t* __restrict__ item_end,
+                                                                 const uint8_t* __restrict__ user_prec, const uint8_t* __restrict__ item_prec,
+                                                                 uint32_t user_groups, uint32_t item_groups, double* sum_sq)
 {
-    constexpr int E = K / 64;
     extern __shared__ __align__(16) uint8_t smem[];
     uint64_t* pptr_s = reinterpret_cast<uint64_t*>(smem);
     uint64_t* qptr_s = pptr_s + user_groups;
@@ -177,46 +273,23 @@ __global__ __launch_bounds__(kBlock) void rmse_grouped_kernel(const mf_node* __r
     for (uint32_t g = threadIdx.x; g < user_groups; g += blockDim.x) { pptr_s[g] = reinterpret_cast<uint64_t>(p[g]); uend_s[g] = user_end[g]; uprec_s[g] = user_prec[g]; }
     for (uint32_t g = threadIdx.x; g < item_groups; g += blockDim.x) { qptr_s[g] = reinterpret_cast<uint64_t>(q[g]); iend_s[g] = item_end[g]; iprec_s[g] = item_prec[g]; }
     __syncthreads();
-    const int lane = threadIdx.x & 63;
-    const uint32_t waves = gridDim.x * kWavesPerBlock;
-    const uint32_t wid = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+    const uint32_t lane = threadIdx.x & 63u;
     double acc = 0;
-    for (uint64_t base = (uint64_t)wid * kWave; base < test_n; base += (uint64_t)waves * kWave) {
-        const uint64_t left = test_n - base;
-        const int n = left < (uint64_t)kWave ? (int)left : kWave;
-        Rating my = {0.f, 0u, 0u};
-        uint64_t pptr = 0, qptr = 0; uint32_t flags = 4u;
-        if (lane < n) {
-            my = load_rating(test, (uint32_t)(base + lane));
-            const uint32_t ug = group_of(uend_s, user_groups, my.u), ig = group_of(iend_s, item_groups, my.v);
-            const bool ok = my.u <= uend_s[ug] && my.v <= iend_s[ig];
-            const uint32_t urow = ug ? my.u - uend_s[ug - 1] - 1 : my.u;
-            const uint32_t irow = ig ? my.v - iend_s[ig - 1] - 1 : my.v;
-            const uint32_t up = uprec_s[ug] ? 1u : 0u, ip = iprec_s[ig] ? 1u : 0u;
-            pptr = pptr_s[ug] + (uint64_t)urow * (K * (up ? 4u : 2u));
-            qptr = qptr_s[ig] + (uint64_t)irow * (K * (ip ? 4u : 2u));
-            flags = up | (ip << 1) | (ok ? 0u : 4u);
-        }
-        for (int j = 0; j < n; ++j) {
-            const uint32_t f = bcast(flags, j);
-            if (f & 4u) continue;
-            const float r = bcast(my.r, j);
-            const uint64_t pa = bcast(pptr, j), qa = bcast(qptr, j);
-            float pv[E], qv[E];
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int el = lane + 64 * e;
-                pv[e] = (f & 1u) ? reinterpret_cast<const float*>(pa)[el] : (float)from_bits<half_t>(reinterpret_cast<const uint16_t*>(pa)[el]);
-                qv[e] = (f & 2u) ? reinterpret_cast<const float*>(qa)[el] : (float)from_bits<half_t>(reinterpret_cast<const uint16_t*>(qa)[el]);
+    for (uint64_t base = ((uint64_t)(threadIdx.x >> 6) * gridDim.x + blockIdx.x) * kWave; base < test_n; base += (uint64_t)gridDim.x * kRmseBlock) {
+        TestRating my = {0.f, 0, 0, 4u};
+        if (base + lane < test_n) {
+            const Rating x = load_rating(test, (uint32_t)(base + lane));
+            const uint32_t ug = group_of(uend_s, user_groups, x.u), ig = group_of(iend_s, item_groups, x.v);
+            if (x.u <= uend_s[ug] && x.v <= iend_s[ig]) {
+                const uint32_t urow = ug ? x.u - uend_s[ug - 1] - 1 : x.u;
+                const uint32_t irow = ig ? x.v - iend_s[ig - 1] - 1 : x.v;
+                const uint32_t up = uprec_s[ug] ? 1u : 0u, ip = iprec_s[ig] ? 1u : 0u;
+                my = {x.r, pptr_s[ug] + (uint64_t)urow * (K * (up ? 4u : 2u)), qptr_s[ig] + (uint64_t)irow * (K * (ip ? 4u : 2u)), up | (ip << 1)};
             }
-            float d = pv[0] * qv[0];
-            if constexpr (E == 2) d = d + pv[1] * qv[1];
-            d = reduce_wave(d, OpAdd());
-            const double err = (double)(r - d);
-            acc += err * err;
         }
+        rmse_wave<K, false>(my, acc);
     }
-    block_sum_to_global(acc, sum_sq);
+    rmse_block_sum(acc, sum_sq);
 }
 
 // ---- model init (model_init.cu:19-28): N(0,1)*0.01 from counter-derived bits ----------------------
@@ -527,9 +600,9 @@ int mf_test_rmse(const mf_node* test, uint32_t test_n, const float* p, const flo
     if (k != 64 && k != 128) return invalid("mf_test_rmse: k must be 64 or 128 (got %d)", k);
     if (test_n == 0) return MF_OK;
     if (!test || !p || !q || !sum_sq) return invalid("mf_test_rmse: null pointer");
-    const uint32_t grid = stream_grid((uint64_t)test_n * 4);
-    if (k == 128) hipLaunchKernelGGL(rmse_dense_kernel<128>, dim3(grid), dim3(kBlock), 0, as_stream(stream), test, test_n, p, q, sum_sq);
-    else hipLaunchKernelGGL(rmse_dense_kernel<64>, dim3(grid), dim3(kBlock), 0, as_stream(stream), test, test_n, p, q, sum_sq);
+    const uint32_t grid = rmse_grid(test_n);
+    if (k == 128) hipLaunchKernelGGL(rmse_dense_kernel<128>, dim3(grid), dim3(kRmseBlock), 0, as_stream(stream), test, test_n, p, q, sum_sq);
+    else hipLaunchKernelGGL(rmse_dense_kernel<64>, dim3(grid), dim3(kRmseBlock), 0, as_stream(stream), test, test_n, p, q, sum_sq);
     return launch_status("mf_test_rmse");
 }
 
@@ -545,9 +618,9 @@ int mf_test_rmse_grouped(const mf_node* test, uint32_t test_n, void* const* p, v
     if (user_group_num == 0 || item_group_num == 0) return invalid("mf_test_rmse_grouped: at least one group per side is required");
     const size_t lds = group_table_lds(user_group_num, item_group_num);
     if (lds > 60 * 1024) return invalid("mf_test_rmse_grouped: group tables need %zu bytes of LDS", lds);
-    const uint32_t grid = stream_grid((uint64_t)test_n * 4);
-    if (k == 128) hipLaunchKernelGGL(rmse_grouped_kernel<128>, dim3(grid), dim3(kBlock), lds, as_stream(stream), test, test_n, p, q, user_group_end_idx, item_group_end_idx, user_group_prec_info, item_group_prec_info, user_group_num, item_group_num, sum_sq);
-    else hipLaunchKernelGGL(rmse_grouped_kernel<64>, dim3(grid), dim3(kBlock), lds, as_stream(stream), test, test_n, p, q, user_group_end_idx, item_group_end_idx, user_group_prec_info, item_group_prec_info, user_group_num, item_group_num, sum_sq);
+    const uint32_t grid = rmse_grid(test_n);
+    if (k == 128) hipLaunchKernelGGL(rmse_grouped_kernel<128>, dim3(grid), dim3(kRmseBlock), lds, as_stream(stream), test, test_n, p, q, user_group_end_idx, item_group_end_idx, user_group_prec_info, item_group_prec_info, user_group_num, item_group_num, sum_sq);
+    else hipLaunchKernelGGL(rmse_grouped_kernel<64>, dim3(grid), dim3(kRmseBlock), lds, as_stream(stream), test, test_n, p, q, user_group_end_idx, item_group_end_idx, user_group_prec_info, item_group_prec_info, user_group_num, item_group_num, sum_sq);
     return launch_status("mf_test_rmse_grouped");
 }
 

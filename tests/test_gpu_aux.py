@@ -404,3 +404,58 @@ def test_workspace_forms_equal_the_allocating_forms(orc):
             assert np.array_equal(from_dev(out, mfutil.NODE).view(np.uint8), want[first:first + count].view(np.uint8))
         with pytest.raises(MfError, match="need"):
             h.mf_synth_build_tables(C.addressof(c), 9, tables.data_ptr(), need - 1, st)
+
+
+# remainders of 64 ratings and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
+# ratings of ids in no group; the sums in binary64 on the host from the same rows (a binary32 dot of k products is off by k / 2^24
+# of the sum of their sizes at most)
+@pytest.mark.parametrize("k", [64, 128])
+@pytest.mark.parametrize("test_n", [1, 63, 64, 65, 16 * 64 + 17, 40_003])
+def test_rmse_gather_mixed_rows(k, test_n):
+    import torch
+    h = mfutil.hip()
+    st = mfutil.stream_ptr()
+    rng = np.random.default_rng(k + test_n)
+    sides = []
+    for end, prec in (([0, 4, 36, 100, 116], [1, 0, 1, 0, 0]), ([6, 7, 50], [0, 1, 0])):
+        rows = end[-1] + 1
+        dense = (rng.standard_normal((rows, k)) * 0.3).astype(np.float32)
+        arena = torch.zeros(rows * k * 4 + 64 * len(end), dtype=torch.uint8, device="cuda")
+        at, ptr, first = 0, [], 0
+        for g, (last, single) in enumerate(zip(end, prec)):
+            at = (at + 15) // 16 * 16 + (4 if single else 2 * (g % 3))      # aligned to elements only
+            part = dense[first:last + 1] if single else dense[first:last + 1].astype(np.float16)
+            dense[first:last + 1] = part
+            raw = torch.from_numpy(part.reshape(-1).view(np.uint8).copy()).cuda()
+            arena[at:at + raw.numel()] = raw
+            ptr.append(arena.data_ptr() + at)
+            at += raw.numel()
+            first = last + 1
+        d = dict(dense=dense, arena=arena, groups=len(end), ptr=torch.tensor(ptr, dtype=torch.int64, device="cuda"),
+                 end=torch.tensor(end, dtype=torch.int32, device="cuda"), prec=torch.tensor(prec, dtype=torch.uint8, device="cuda"))
+        out = torch.full(((rows + 1) * k,), 9.0, dtype=torch.float32, device="cuda")
+        h.mf_grouped_params2dense(d["ptr"].data_ptr(), d["end"].data_ptr(), d["prec"].data_ptr(), out.data_ptr(), k, rows, len(end), st)
+        _sync()
+        assert np.array_equal(out[:rows * k].cpu().numpy().reshape(rows, k), dense) and bool((out[rows * k:] == 9.0).all())
+        sides.append(d)
+    U, I = sides
+    T = np.zeros(test_n, mfutil.NODE)
+    T["u"], T["i"], T["r"] = rng.integers(0, U["dense"].shape[0], test_n), rng.integers(0, I["dense"].shape[0], test_n), rng.random(test_n) * 4 + 1
+    acc = torch.zeros(1, dtype=torch.float64, device="cuda")
+    for outside in (False, True):
+        if outside:
+            T["u"][::3] = U["dense"].shape[0] + 5
+        ok = T["u"] < U["dense"].shape[0]
+        P, Q = U["dense"][np.where(ok, T["u"], 0)].astype(np.float64), I["dense"][T["i"]].astype(np.float64)
+        err = np.where(ok, T["r"].astype(np.float64) - (P * Q).sum(1), 0.0)
+        bound = (2 * np.abs(err) * (np.abs(P * Q).sum(1) * k + 8) * 2.0 ** -24).sum() + 1e-12
+        dT = to_dev(T)
+        acc.zero_()
+        h.mf_test_rmse_grouped(dT.data_ptr(), test_n, U["ptr"].data_ptr(), I["ptr"].data_ptr(), k, U["end"].data_ptr(), I["end"].data_ptr(), U["prec"].data_ptr(), I["prec"].data_ptr(),
+                               U["groups"], I["groups"], acc.data_ptr(), st)
+        assert abs(float(acc) - (err ** 2).sum()) <= bound
+        if not outside:
+            dP, dQ = to_dev(U["dense"]), to_dev(I["dense"])
+            acc.zero_()
+            h.mf_test_rmse(dT.data_ptr(), test_n, dP.data_ptr(), dQ.data_ptr(), k, acc.data_ptr(), st)
+            assert abs(float(acc) - (err ** 2).sum()) <= bound
