@@ -406,6 +406,33 @@ def test_workspace_forms_equal_the_allocating_forms(orc):
             h.mf_synth_build_tables(C.addressof(c), 9, tables.data_ptr(), need - 1, st)
 
 
+# ids in one range of the counting kernel (80896), across two, in the item range behind the users', past every range, and
+# counters that pass 2^15 several times
+@pytest.mark.parametrize("n,n_users,n_items,hot", [(1, 1, 1, False), (63, 80895, 1, False), (16385, 80896, 80897, False), (70_001, 3, 90_000, True),
+                                                   (300_007, 161_793, 161_000, True), (900_001, 3_000_000, 700_000, True), (400_003, 10, 5_000_000, False)])
+def test_histogram_reindex_ranges(n, n_users, n_items, hot):
+    import torch
+    h = mfutil.hip()
+    rng = np.random.default_rng(n)
+    R = np.zeros(n, mfutil.NODE)
+    R["u"], R["i"], R["r"] = rng.integers(0, n_users, n), rng.integers(0, n_items, n), rng.random(n)
+    if hot:
+        R["u"][rng.random(n) < 0.6] = n_users - 1
+        R["i"][rng.random(n) < 0.3] = n_items // 2
+    ub = torch.full((n_users,), 7, dtype=torch.int32, device="cuda")       # counts are added to what is there
+    ib = torch.zeros(n_items, dtype=torch.int32, device="cuda")
+    dR = to_dev(R)
+    h.mf_user_item_histogram(dR.data_ptr(), n, ub.data_ptr(), ib.data_ptr(), mfutil.stream_ptr())
+    u2s, i2s = rng.permutation(n_users).astype(np.uint32), rng.permutation(n_items).astype(np.uint32)
+    d_u2s, d_i2s = to_dev(u2s), to_dev(i2s)
+    h.mf_matrix_reconst_triplet(dR.data_ptr(), d_u2s.data_ptr(), d_i2s.data_ptr(), n, mfutil.stream_ptr())
+    _sync()
+    assert np.array_equal(ub.cpu().numpy(), np.bincount(R["u"], minlength=n_users) + 7)
+    assert np.array_equal(ib.cpu().numpy(), np.bincount(R["i"], minlength=n_items))
+    got = from_dev(dR, mfutil.NODE)
+    assert np.array_equal(got["r"], R["r"]) and np.array_equal(got["u"], u2s[R["u"]]) and np.array_equal(got["i"], i2s[R["i"]])
+
+
 # remainders of 64 ratings and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
 # ratings of ids in no group; the sums in binary64 on the host from the same rows (a binary32 dot of k products is off by k / 2^24
 # of the sum of their sizes at most)
