@@ -466,7 +466,11 @@ __global__ __launch_bounds__(kStreamBlock) void iota_kernel(uint32_t* __restrict
 // counters would take percents of them.  User and item ids are laid end to end and cut into ranges of kHistBins; the
 // workgroups of one chunk sit on one XCD, so that its L2 hands them the same ratings.  How far the ids reach is not
 // an argument: every workgroup takes the largest ids of the same kHistSample ratings, spread over the input, and the few
-// above them (and those past kHistRanges ranges) are added in memory by the workgroup of the first range.
+// above them are added in memory by the workgroups of the first and the last range.
+// Ids that reach further than kHistRanges ranges are counted in a hash table in LDS instead, kHistSlots (id, count) slots per
+// side, a slot claimed by the first id that hashes to it (two probes); ids that find both taken go to memory.  At
+// 100M ratings the ranges take 1.5 ms for 15 of them whatever the popularity is, and from 17 on, with one chunk per XCD, they would take 3; the table takes 3.3 ms for 250M ratings of 1M + 625k ids under Zipf(1.2), where nearly all ids find a slot,
+// 6.1 for 100M under Zipf(0.8) (tables half as large, in smaller workgroups: 4.1 and 6.9).
 // What bounds it is the L1 and the instructions per id: each range's workgroup reads the whole chunk.  100M ratings over 480k + 17.8k ids: 0.84 ms
 // (0.97 with every result looked at by itself, 1.63 without the next tile's loads in flight); with a 4096-entry hash table per
 // side and workgroup, which sends two thirds of the user counts to memory, about 4.2.
@@ -476,10 +480,12 @@ __global__ __launch_bounds__(kStreamBlock) void iota_kernel(uint32_t* __restrict
 constexpr int kHistBlock = 1024;
 constexpr uint32_t kHistUnroll = 16;
 constexpr uint32_t kHistHalf = 40448, kHistBins = 2 * kHistHalf;      // words, each the counters of ids x and x + kHistHalf of the range
-constexpr uint32_t kHistRanges = 32, kHistGrid = 256;                 // one workgroup per compute unit, 32 per XCD
+constexpr uint32_t kHistRanges = 16, kHistGrid = 256;                 // one workgroup per compute unit, 32 per XCD
+constexpr uint32_t kHistLog = 13, kHistSlots = 1u << kHistLog;
 constexpr uint32_t kHistSample = 4 * kHistBlock;
 constexpr uint32_t kHistChunkMin = 1u << 14;                          // ratings: below, emptying the counters costs more than counting
 constexpr size_t kHistLds = (size_t)kHistHalf * 4;
+static_assert(4 * kHistSlots <= kHistHalf, "the hash tables fit where the counters are");
 static_assert(kHistBlock * kHistUnroll + 0x8000u < 0x10000u, "a 16-bit counter cannot overflow between two barriers");
 struct HistogramRange {
     uint32_t* bin;            // LDS
@@ -519,6 +525,45 @@ struct HistogramRange {
         }
     }
 };
+__device__ __forceinline__ void hashed_count(uint32_t* tag, uint32_t* cnt, uint32_t id, uint32_t* global_bin)
+{
+    uint32_t s = (id * 2654435761u) >> (32 - kHistLog);
+#pragma unroll
+    for (int probe = 0; probe < 2; ++probe, s ^= 1u) {
+        uint32_t t = tag[s];
+        if (t == 0u) t = atomicCAS(&tag[s], 0u, id + 1u);
+        if (t == 0u || t == id + 1u) { atomicAdd(&cnt[s], 1u); return; }
+    }
+    atomicAdd(&global_bin[id], 1u);
+}
+// tab: 4 * kHistSlots words of LDS, zero
+__device__ __forceinline__ void histogram_hashed(const mf_node* __restrict__ R, uint32_t n, uint32_t* user_bin, uint32_t* item_bin, uint32_t* tab)
+{
+    uint32_t* utag = tab, *ucnt = tab + kHistSlots, *itag = tab + 2 * kHistSlots, *icnt = tab + 3 * kHistSlots;
+    const uint64_t begin = (uint64_t)n * blockIdx.x / kHistGrid, end = (uint64_t)n * (blockIdx.x + 1u) / kHistGrid;
+    constexpr uint32_t kAhead = 8;
+    for (uint64_t base = begin; base < end; base += kHistBlock * kAhead) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(R + base);
+        const uint32_t left = end - base < kHistBlock * kAhead ? (uint32_t)(end - base) : kHistBlock * kAhead;
+        uint32_t u[kAhead], v[kAhead];
+#pragma unroll
+        for (uint32_t j = 0; j < kAhead; ++j) {
+            const uint32_t o = min(j * kHistBlock + threadIdx.x, left - 1u) * 3u;
+            u[j] = __builtin_nontemporal_load(w + o + 1u); v[j] = __builtin_nontemporal_load(w + o + 2u);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kAhead; ++j) {
+            if (j * kHistBlock + threadIdx.x >= left) continue;
+            hashed_count(utag, ucnt, u[j], user_bin);
+            hashed_count(itag, icnt, v[j], item_bin);
+        }
+    }
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s < kHistSlots; s += kHistBlock) {
+        if (utag[s]) atomicAdd(&user_bin[utag[s] - 1u], ucnt[s]);
+        if (itag[s]) atomicAdd(&item_bin[itag[s] - 1u], icnt[s]);
+    }
+}
 __global__ __launch_bounds__(kHistBlock) void histogram_kernel(const mf_node* __restrict__ R, uint32_t n, uint32_t* user_bin, uint32_t* item_bin)
 {
     extern __shared__ uint32_t hist_bin[];
@@ -534,12 +579,13 @@ __global__ __launch_bounds__(kHistBlock) void histogram_kernel(const mf_node* __
     }
     atomicMax(&reach[0], mu); atomicMax(&reach[1], mv);
     __syncthreads();
-    const uint32_t most = kHistRanges / 2 * kHistBins;
+    const uint32_t most = (kHistRanges + 1u) * kHistBins;
     const uint32_t users = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(reach[0], most - 1u)) + 1u;
     const uint32_t items = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(reach[1], most - 1u)) + 1u;
     // the items begin a range of their own where that takes no more ranges: then no workgroup reads both ids
     const uint32_t user_ranges = (users + kHistBins - 1u) / kHistBins, apart = user_ranges + (items + kHistBins - 1u) / kHistBins;
-    const uint32_t ranges = (users + items + kHistBins - 1u) / kHistBins;          // <= kHistRanges
+    const uint32_t ranges = (users + items + kHistBins - 1u) / kHistBins;
+    if (ranges > kHistRanges) { histogram_hashed(R, n, user_bin, item_bin, hist_bin); return; }
     const uint32_t item_base = apart == ranges ? user_ranges * kHistBins : users;
     const uint32_t xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
     const uint32_t per_xcd = kHistGrid / kXcds / ranges, by_size = n / kHistChunkMin + 1u;

@@ -406,10 +406,10 @@ def test_workspace_forms_equal_the_allocating_forms(orc):
             h.mf_synth_build_tables(C.addressof(c), 9, tables.data_ptr(), need - 1, st)
 
 
-# ids in one range of the counting kernel (80896), across two, in the item range behind the users', past every range, and
+# ids in one range of the counting kernel (80896), across two, in the item ranges behind the users', in 15 ranges, in too many for it, and
 # counters that pass 2^15 several times
 @pytest.mark.parametrize("n,n_users,n_items,hot", [(1, 1, 1, False), (63, 80895, 1, False), (16385, 80896, 80897, False), (70_001, 3, 90_000, True),
-                                                   (300_007, 161_793, 161_000, True), (900_001, 3_000_000, 700_000, True), (400_003, 10, 5_000_000, False)])
+                                                   (300_007, 161_793, 161_000, True), (900_001, 3_000_000, 700_000, True), (500_001, 1_000_000, 200_000, True), (400_003, 10, 5_000_000, False)])
 def test_histogram_reindex_ranges(n, n_users, n_items, hot):
     import torch
     h = mfutil.hip()
