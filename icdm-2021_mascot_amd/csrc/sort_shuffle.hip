@@ -19,8 +19,10 @@ namespace mf {
 //   finish    one workgroup per bucket: ordered by the next 12 bits of the key, ties by the whole key, written in order
 // What bounds it is memory traffic: 16 bytes written, read and written again, read, and 12 bytes written.  A radix sort of
 // (key, position) pairs moved 24 bytes eight times and then gathered the ratings from random places, a cache line for
-// each 12 bytes: at 100M ratings 9.7 ms, of which the gather took 2.7; this takes 2.8 (the two partition passes 0.88 each,
-// at 3.4 TB/s, the counts 0.35, the finish 0.67).
+// each 12 bytes: at 100M ratings 9.7 ms, of which the gather took 2.7; this takes 2.6 (the two partition passes 0.76 and 0.75,
+// at 3.7 and 4.3 TB/s, the counts 0.45, the finish 0.65).  Rating and position move as one 16-byte record: in two arrays the
+// partition passes took 0.88 each, a lane's two stores ending in twice as many partly written lines (the second count, which
+// reads positions alone, 0.1 less).
 constexpr int kShufBlock = 512;                   // the placing and the finishing kernel
 constexpr uint32_t kPerThread = 8;
 constexpr uint32_t kBucketCap = kShufBlock * kPerThread;      // ratings that the finishing workgroup orders in LDS
@@ -54,13 +56,21 @@ template <int BLOCK> __device__ __forceinline__ void block_scan(uint32_t* v, uin
     __syncthreads();
 }
 
+// A rating and its position, where they have been moved together, or from the original order.  Which it is is known at compile
+// time: with a branch between them every load would be waited for before the next.
+template <bool MOVED> __device__ __forceinline__ uint4 record(const uint4* moved, const Node3* nodes, uint32_t at)
+{
+    if constexpr (MOVED) return moved[at];
+    const Node3 x = nodes[at];
+    return make_uint4(x.r, x.u, x.i, at);
+}
+
 // What a workgroup of a pass works on: ratings [begin, end) of the input, which all belong to segment `seg` (one segment,
 // the whole input, in the first pass; the first pass's buckets in the second), as chunk `chunk` of that segment.
 struct PassArgs {
-    const uint32_t* idx;          // positions of the input ratings, null: the input is in its original order
-    const Node3* nodes;
-    uint32_t* idx_out;
-    Node3* nodes_out;
+    const Node3* nodes;           // the first pass's input
+    const uint4* moved;           // the second's: a rating and its position; null in the first pass
+    uint4* moved_out;
     uint32_t n; uint64_t base;
     int skip, bits;               // the digit of this pass
     uint32_t chunks;              // workgroups per segment
@@ -89,7 +99,7 @@ template <int BLOCK> __global__ __launch_bounds__(BLOCK) void shuffle_count_kern
     chunk_of<BLOCK * kPerThread>(a, seg, begin, end);
 #pragma unroll 4
     for (uint64_t i = (uint64_t)begin + threadIdx.x; i < end; i += BLOCK) {
-        const uint32_t pos = a.idx ? a.idx[i] : (uint32_t)i;
+        const uint32_t pos = a.moved ? a.moved[i].w : (uint32_t)i;
         atomicAdd(&cnt[key_digit(mix64(a.base ^ (uint64_t)pos), a.skip, a.bits)], 1u);
     }
     __syncthreads();
@@ -143,7 +153,7 @@ static size_t place_lds(int bits) { const size_t bins = (size_t)1 << bits; retur
 // 16 wavefronts on a compute unit, each lane with 8 ratings in flight: one workgroup of 1024 threads (147 KB of LDS) up to
 // 256 digits, two of 512 above.  The larger tile writes runs twice as long, and with half as many workgroups the cache lines
 // that are partly written at any time fit in an XCD's L2.
-template <int BLOCK> __global__ __launch_bounds__(BLOCK) void shuffle_partition_kernel(PassArgs a)
+template <int BLOCK, bool MOVED> __global__ __launch_bounds__(BLOCK) void shuffle_partition_kernel(PassArgs a)
 {
     constexpr uint32_t kTile = BLOCK * kPerThread;
     extern __shared__ __align__(16) uint32_t shuf_smem[];
@@ -156,13 +166,12 @@ template <int BLOCK> __global__ __launch_bounds__(BLOCK) void shuffle_partition_
     for (uint32_t d = threadIdx.x; d < bins; d += BLOCK) next[d] = a.table[(size_t)blockIdx.x * bins + d];
     uint32_t seg, begin, end;
     chunk_of<kTile>(a, seg, begin, end);
-    Node3 node[kPerThread]; uint32_t pos[kPerThread];
-    auto fetch = [&](uint64_t tile) {
+    uint4 rec[kPerThread];
+    auto fetch = [&](uint64_t tile) {      // without a branch per load, which would be waited for; past the end the last rating again
+        if (tile >= end) return;
+        const uint32_t most = end - tile < kTile ? (uint32_t)(end - tile) - 1u : kTile - 1u;
 #pragma unroll
-        for (uint32_t j = 0; j < kPerThread; ++j) {
-            const uint64_t o = tile + j * BLOCK + threadIdx.x;
-            if (o < end) { node[j] = a.nodes[o]; pos[j] = a.idx ? a.idx[o] : (uint32_t)o; }
-        }
+        for (uint32_t j = 0; j < kPerThread; ++j) rec[j] = record<MOVED>(a.moved, a.nodes, (uint32_t)tile + min(j * BLOCK + threadIdx.x, most));
     };
     fetch(begin);
     for (uint64_t tile = begin; tile < end; tile += kTile) {
@@ -173,7 +182,7 @@ template <int BLOCK> __global__ __launch_bounds__(BLOCK) void shuffle_partition_
 #pragma unroll
         for (uint32_t j = 0; j < kPerThread; ++j) {
             if (j * BLOCK + threadIdx.x < m) {
-                digit[j] = key_digit(mix64(a.base ^ (uint64_t)pos[j]), a.skip, a.bits);
+                digit[j] = key_digit(mix64(a.base ^ (uint64_t)rec[j].w), a.skip, a.bits);
                 rank[j] = atomicAdd(&cnt[digit[j]], 1u);
             }
         }
@@ -183,7 +192,7 @@ template <int BLOCK> __global__ __launch_bounds__(BLOCK) void shuffle_partition_
         for (uint32_t j = 0; j < kPerThread; ++j) {
             if (j * BLOCK + threadIdx.x < m) {
                 const uint32_t at = cnt[digit[j]] + rank[j];
-                stage[at] = make_uint4(node[j].r, node[j].u, node[j].i, pos[j]);
+                stage[at] = rec[j];
                 digit_of[at] = (uint16_t)digit[j];
             }
         }
@@ -193,11 +202,8 @@ template <int BLOCK> __global__ __launch_bounds__(BLOCK) void shuffle_partition_
         for (uint32_t j = 0; j < kPerThread; ++j) {
             const uint32_t o = j * BLOCK + threadIdx.x;
             if (o < m) {
-                const uint4 x = stage[o];
-                const uint32_t d = digit_of[o], to = next[d] + (o - cnt[d]);
-                Node3 y; y.r = x.x; y.u = x.y; y.i = x.z;
-                a.nodes_out[to] = y;
-                a.idx_out[to] = x.w;
+                const uint32_t d = digit_of[o];
+                a.moved_out[next[d] + (o - cnt[d])] = stage[o];
             }
         }
         __syncthreads();
@@ -210,7 +216,8 @@ static size_t partition_lds(int bits) { const size_t tile = (bits <= kLargeTileB
 
 // One bucket in order: by the kSubBits bits of the key after the bucket's, in LDS (0.75 ratings per value on average), then by
 // the whole key among the ratings that share them.  64 KB of LDS: two workgroups per compute unit.
-__global__ __launch_bounds__(kShufBlock) void shuffle_finish_kernel(const uint32_t* __restrict__ idx, const Node3* __restrict__ nodes, Node3* __restrict__ out,
+template <bool MOVED>
+__global__ __launch_bounds__(kShufBlock) void shuffle_finish_kernel(const uint4* __restrict__ moved, const Node3* __restrict__ nodes, Node3* __restrict__ out,
                                                                     uint32_t n, uint64_t base, int skip, const uint32_t* __restrict__ bucket_start, uint32_t buckets)
 {
     __shared__ uint32_t first[kSubBins];
@@ -220,25 +227,24 @@ __global__ __launch_bounds__(kShufBlock) void shuffle_finish_kernel(const uint32
     const uint32_t m = end - begin;
     if (m > kBucketCap) {       // larger than the LDS: each rating's place is counted out
         for (uint32_t o = threadIdx.x; o < m; o += kShufBlock) {
-            const uint64_t key = mix64(base ^ (uint64_t)(idx ? idx[begin + o] : begin + o));
+            const uint4 x = record<MOVED>(moved, nodes, begin + o);
+            const uint64_t key = mix64(base ^ (uint64_t)x.w);
             uint32_t rank = 0;
-            for (uint32_t q = 0; q < m; ++q) rank += mix64(base ^ (uint64_t)(idx ? idx[begin + q] : begin + q)) < key ? 1u : 0u;
-            out[begin + rank] = nodes[begin + o];
+            for (uint32_t q = 0; q < m; ++q) rank += mix64(base ^ (uint64_t)record<MOVED>(moved, nodes, begin + q).w) < key ? 1u : 0u;
+            out[begin + rank] = Node3{x.x, x.y, x.z};
         }
         return;
     }
+    if (m == 0u) return;
     for (uint32_t d = threadIdx.x; d < kSubBins; d += kShufBlock) first[d] = 0u;
-    Node3 node[kPerThread]; uint64_t key[kPerThread]; uint32_t place[kPerThread];
+    uint4 rec[kPerThread]; uint64_t key[kPerThread]; uint32_t place[kPerThread];
 #pragma unroll
-    for (uint32_t j = 0; j < kPerThread; ++j) {
-        const uint32_t o = j * kShufBlock + threadIdx.x;
-        if (o < m) { key[j] = idx ? idx[begin + o] : begin + o; node[j] = nodes[begin + o]; }
-    }
+    for (uint32_t j = 0; j < kPerThread; ++j) rec[j] = record<MOVED>(moved, nodes, begin + min(j * kShufBlock + threadIdx.x, m - 1u));
     __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < kPerThread; ++j) {
         if (j * kShufBlock + threadIdx.x < m) {
-            key[j] = mix64(base ^ key[j]);
+            key[j] = mix64(base ^ (uint64_t)rec[j].w);
             place[j] = atomicAdd(&first[key_digit(key[j], skip, kSubBits)], 1u);
         }
     }
@@ -261,7 +267,7 @@ __global__ __launch_bounds__(kShufBlock) void shuffle_finish_kernel(const uint32
     __syncthreads();
 #pragma unroll
     for (uint32_t j = 0; j < kPerThread; ++j)
-        if (j * kShufBlock + threadIdx.x < m) { stage[place[j] * 3] = node[j].r; stage[place[j] * 3 + 1] = node[j].u; stage[place[j] * 3 + 2] = node[j].i; }
+        if (j * kShufBlock + threadIdx.x < m) { stage[place[j] * 3] = rec[j].x; stage[place[j] * 3 + 1] = rec[j].y; stage[place[j] * 3 + 2] = rec[j].z; }
     __syncthreads();
     uint32_t* to = reinterpret_cast<uint32_t*>(out + begin);
     for (uint32_t w = threadIdx.x; w < m * 3; w += kShufBlock) to[w] = stage[w];
@@ -301,7 +307,7 @@ static int sort_in(uint32_t* cnt, uint32_t* idx, uint32_t n, uint8_t* ws, size_t
 struct ShufflePlan {
     int bits1 = 0, bits2 = 0;
     uint32_t chunks1 = 0, chunks2 = 0;
-    size_t idx[2], nodes[2], table[2], start[2], total = 0;
+    size_t moved[2], table[2], start[2], total = 0;
 };
 static ShufflePlan shuffle_plan(uint32_t n)
 {
@@ -322,8 +328,7 @@ static ShufflePlan shuffle_plan(uint32_t n)
     for (int l = 0; l < 2; ++l) {
         const int b = l ? p.bits2 : p.bits1;
         if (!b) continue;
-        p.idx[l] = take((size_t)n * 4);
-        p.nodes[l] = take((size_t)n * sizeof(Node3));
+        p.moved[l] = take((size_t)n * sizeof(uint4));
         p.table[l] = take(l ? (((size_t)p.chunks2 << p.bits1) << p.bits2) * 4 : ((size_t)p.chunks1 << p.bits1) * 4);
         p.start[l] = take(((size_t)1 << (l ? p.bits1 + p.bits2 : p.bits1)) * 4);
     }
@@ -425,9 +430,8 @@ int mf_shuffle_ratings_ws(const mf_node* in, mf_node* out, uint32_t n, uint64_t 
         a.bits = l ? p.bits2 : p.bits1;
         if (!a.bits) break;
         a.chunks = l ? p.chunks2 : p.chunks1;
-        a.idx_out = reinterpret_cast<uint32_t*>(ws + p.idx[l]); a.nodes_out = reinterpret_cast<Node3*>(ws + p.nodes[l]);
+        a.moved_out = reinterpret_cast<uint4*>(ws + p.moved[l]);
         a.table = reinterpret_cast<uint32_t*>(ws + p.table[l]); a.bucket_start = reinterpret_cast<uint32_t*>(ws + p.start[l]);
-        const dim3 grid(a.segs * a.chunks), block(kShufBlock);
         auto pass = [&](auto Block, auto count, auto partition) -> int {
             const dim3 grid(a.segs * a.chunks), block(decltype(Block)::value);
             if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(partition), hipFuncAttributeMaxDynamicSharedMemorySize, (int)partition_lds(a.bits)),
@@ -437,13 +441,17 @@ int mf_shuffle_ratings_ws(const mf_node* in, mf_node* out, uint32_t n, uint64_t 
             hipLaunchKernelGGL(partition, grid, block, partition_lds(a.bits), s, a);
             return MF_OK;
         };
-        if (int rc = a.bits <= kLargeTileBits ? pass(std::integral_constant<int, 1024>(), shuffle_count_kernel<1024>, shuffle_partition_kernel<1024>)
-                                              : pass(std::integral_constant<int, 512>(), shuffle_count_kernel<512>, shuffle_partition_kernel<512>)) return rc;
+        auto either = [&](auto Moved) {
+            constexpr bool moved = decltype(Moved)::value;
+            return a.bits <= kLargeTileBits ? pass(std::integral_constant<int, 1024>(), shuffle_count_kernel<1024>, shuffle_partition_kernel<1024, moved>)
+                                            : pass(std::integral_constant<int, 512>(), shuffle_count_kernel<512>, shuffle_partition_kernel<512, moved>);
+        };
+        if (int rc = l ? either(std::true_type()) : either(std::false_type())) return rc;
         if (int rc = launch_status("mf_shuffle_ratings: partition")) return rc;
-        a.idx = a.idx_out; a.nodes = a.nodes_out; a.seg_start = a.bucket_start;
+        a.moved = a.moved_out; a.seg_start = a.bucket_start;
         a.segs <<= a.bits; a.skip += a.bits;
     }
-    hipLaunchKernelGGL(shuffle_finish_kernel, dim3(a.segs), dim3(kShufBlock), 0, s, a.idx, a.nodes, reinterpret_cast<Node3*>(out), n, a.base, a.skip, a.seg_start, a.segs);
+    hipLaunchKernelGGL((a.moved ? shuffle_finish_kernel<true> : shuffle_finish_kernel<false>), dim3(a.segs), dim3(kShufBlock), 0, s, a.moved, a.nodes, reinterpret_cast<Node3*>(out), n, a.base, a.skip, a.seg_start, a.segs);
     return launch_status("mf_shuffle_ratings: order");
 }
 int mf_shuffle_ratings(const mf_node* in, mf_node* out, uint32_t n, uint64_t seed, void* stream)
