@@ -13,6 +13,7 @@ inline int check_hip(hipError_t e, const char* what)
 {
     if (e == hipSuccess) return MF_OK;
     set_error("%s: %s", what, hipGetErrorString(e));
+    (void)hipGetLastError();      // reported here: the runtime keeps it, and the next launch's check (or another library's) would take it for its own
     return (int)e;
 }
 inline int launch_status(const char* what) { return check_hip(hipGetLastError(), what); }

@@ -15,10 +15,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <memory>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 #include "mf_host.h"
@@ -94,7 +94,7 @@ public:
     IdCheck(const Common& c, const mf_node* R, const mf_node* test) : c(c), set{R, test}, n{c.n, c.test_n}
     {
         try { worker = std::thread([this] { run(); }); }
-        catch (const std::system_error&) { run(); }      // no thread to be had
+        catch (const std::exception&) { run(); }      // no thread to be had, or no memory for one
     }
     ~IdCheck() { wait(); }
     IdCheck(const IdCheck&) = delete;

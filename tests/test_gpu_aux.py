@@ -79,6 +79,22 @@ def test_empty_inputs_are_no_ops():
     assert h.mf_shuffle_ratings(None, None, 0, 1, None) == 0
 
 
+def test_a_failed_call_leaves_no_error_behind():
+    """The runtime keeps the last error until it is asked for it.  A model that no card can hold is refused by hipMalloc, before
+    anything is launched; the calls after it, of this library and of torch, must not find that error."""
+    import ctypes as C
+    import torch
+    from importlib import import_module
+    MfError = import_module("icdm-2021_mascot_amd.capi").MfError
+    h = mfutil.hip()
+    node, model, out = np.zeros(1, mfutil.NODE), np.zeros(128, np.float32), C.c_double(0)
+    with pytest.raises(MfError, match=r"hipMalloc\(P\)"):
+        h.mf_gpu_test_rmse(node.ctypes.data, 1, model.ctypes.data, model.ctypes.data, 0xffffffff, 1, 128, C.addressof(out))
+    idx = torch.zeros(100, dtype=torch.int32, device="cuda")
+    h.mf_init_idx_arr(idx.data_ptr(), 100, mfutil.stream_ptr())
+    assert idx.sum().item() == 4950
+
+
 def _preprocess_reference(orc, R, n_users, n_items, ug_req, ig_req):
     uc, ic = orc.histogram(R, n_users, n_items)
     suc, sui = orc.sort_by_count(uc)
