@@ -28,32 +28,40 @@ sys.path.insert(0, ROOT)
 PEAK_HBM_GBS = 8000.0
 TRAIN = dict(epochs=50, lr=0.01, decay=0.1, lam=0.015, sample_ratio=0.05, interval=2, ug=100, ig=100, threshold=20.0)
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE of a plain epoch's update kernels, recorded with the workload and the digest of
-# the kernel sources they were taken with; reported only for that workload and those sources
+# the kernel sources and compiler flags they were taken with; reported only for that workload and that build
 PROFILED_TRAFFIC = os.path.join(ROOT, "profiles", "hogwild_mascot_k128_config4_hbm_traffic.json")
 KERNEL_SOURCES = os.path.join(ROOT, "icdm-2021_mascot_amd", "csrc")
+BUILD_FLAGS = importlib.import_module("icdm-2021_mascot_amd.build").FLAGS_RECORD
 
 
-def kernel_sources_digest():
-    """sha256 over the sources of the library (file names and contents, in name order): the kernels, and the host code
-    whose defaults decide how rows are treated."""
+def kernel_build_digest():
+    """sha256 over the sources of the library (file names and contents, in name order: the kernels, and the host code whose
+    defaults decide how rows are treated) and the compiler flags its build recorded, which decide which stores and waits the
+    kernels are made of; None when there is no such record."""
     h = hashlib.sha256()
     for name in sorted(os.listdir(KERNEL_SOURCES)):
         if name.endswith((".h", ".hip", ".cpp")):
             h.update(name.encode())
             with open(os.path.join(KERNEL_SOURCES, name), "rb") as f:
                 h.update(f.read())
+    try:
+        with open(BUILD_FLAGS, "rb") as f:
+            h.update(f.read())
+    except OSError:
+        return None
     return h.hexdigest()
 
 
 def profiled_traffic(config, n_train, k, seed, workers):
     """The committed HBM-side bytes per plain epoch of this workload, or None when the record is of another workload or
-    of other kernel sources than the ones this library was built from."""
+    of another build than this library's."""
     try:
         rec = json.load(open(PROFILED_TRAFFIC))
     except (OSError, ValueError):
         return None
     same = (rec.get("config"), rec.get("n_train"), rec.get("k"), rec.get("seed"), rec.get("workers")) == (config, n_train, k, seed, workers)
-    if not same or rec.get("kernel_sources_sha256") != kernel_sources_digest():
+    digest = kernel_build_digest()
+    if not same or digest is None or rec.get("kernel_build_sha256") != digest:
         return None
     return rec
 

@@ -11,6 +11,7 @@ OBJ = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libmascot_hip.so")
 CLI = os.path.join(HERE, "quantized_mf")
 EVAL = os.path.join(HERE, "test_mf")
+FLAGS_RECORD = os.path.join(OBJ, "device_flags.txt")      # what the library beside it was compiled with, a line per translation unit
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -48,9 +49,18 @@ def _run(cmd):
     return out
 
 
+def device_flags(src):
+    """The compiler flags of one .hip file."""
+    return DEVICE_FLAGS
+
+
+def flags_record():
+    return "".join("%s: %s\n" % (src, " ".join(device_flags(src))) for src in sorted(KERNEL_SOURCES))
+
+
 def _compile(src):
     obj = os.path.join(OBJ, os.path.splitext(src)[0] + ".o")
-    flags = DEVICE_FLAGS if src.endswith(".hip") else ["-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include"]
+    flags = device_flags(src) if src.endswith(".hip") else ["-O2", "-std=c++17", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include"]
     _run([HIPCC] + flags + ["-c", os.path.join(CSRC, src), "-o", obj])
     return obj
 
@@ -60,7 +70,11 @@ def build(verbose=False):
     lib_sources = [s for s in KERNEL_SOURCES + HOST_SOURCES if os.path.exists(os.path.join(CSRC, s))]
     with ThreadPoolExecutor(max_workers=8) as ex:
         objs = list(ex.map(_compile, lib_sources))
+    if os.path.exists(FLAGS_RECORD):
+        os.remove(FLAGS_RECORD)      # none while it may not be the library's
     _run([HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", LIB] + objs)
+    with open(FLAGS_RECORD, "w") as f:
+        f.write(flags_record())
     if all(os.path.exists(os.path.join(CSRC, s)) for s in CLI_SOURCES):
         with ThreadPoolExecutor(max_workers=2) as ex:
             cobjs = list(ex.map(_compile, CLI_SOURCES))
