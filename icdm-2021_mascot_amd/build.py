@@ -21,21 +21,33 @@ ARCH = "gfx950"
 # fma-mix-insts disabled: v_fma_mix{lo,hi}_f16 rounds fma(a,b,c) once to binary16, but the update rules
 # round to binary32 first and then to binary16 (fmaf followed by __float2half); the two differ by one
 # binary16 ulp on rare inputs, so the fused form must not be selected.
+DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-munsafe-fp-atomics",
+                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                "-Xclang", "-target-feature", "-Xclang", "-fma-mix-insts", "-Wall", "-Wno-unused-function"]
 # -structurizecfg-skip-uniform-regions: the update kernels branch on wave-uniform values (how a row is written, the
 # precisions of a rating's rows).  By default the compiler structurises those branches as if lanes could disagree: flag
 # registers, three branches for a three-way choice, and paths on which no store is issued, so that the waits for row
 # loads must assume the fewest stores in between.  Without it a MASCOT rating waits at vmcnt(12..13) instead of (6..7)
-# with a dozen scalar instructions fewer: an epoch of 8M ratings takes 4.74 instead of 5.73 ms, one of 100M 11.13
-# instead of 11.31.
+# with a dozen scalar instructions fewer.
 # -enable-tail-merge=false goes with it: a device-scope store and a cached store of the same registers are one
 # instruction until their cache policies are filled in, and merged they become a device-scope store, which for the copies of
-# replicated rows serialises at the memory side.
-DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-munsafe-fp-atomics",
-                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-                "-Xclang", "-target-feature", "-Xclang", "-fma-mix-insts", "-Wall", "-Wno-unused-function",
-                "-mllvm", "-structurizecfg-skip-uniform-regions=true", "-mllvm", "-enable-tail-merge=false"] + os.environ.get("MF_HIPCC_FLAGS", "").split()
-KERNEL_SOURCES = ["launch_mascot_plain.hip", "launch_mascot_sampled.hip", "launch_mascot_binary16.hip", "launch_muppet.hip", "launch_afp.hip", "hogwild_launch.hip", "launch_mem_quant.hip", "aux_kernels.hip",
-                  "sort_shuffle.hip", "launch_mascot.hip"]
+# replicated rows serialises at the memory side (an epoch of 250M ratings in 121 ms instead of 28).
+# Epochs without -> with the two flags, both libraries in turn on one model (ms; runs of one side differ by 0.1 to 0.5 %):
+#                        k = 64: 8M      100M              k = 128: 8M      100M
+#   MASCOT, all binary16   5.37 -> 5.19   8.36 -> 8.20        5.81 -> 4.75   11.29 -> 11.08
+#   MASCOT, 10 % binary32  6.43 -> 5.94  10.46 -> 9.81        7.58 -> 6.08   15.88 -> 15.71
+#   -v 7                   5.27 -> 5.09   8.11 -> 8.00        5.92 -> 4.88   11.85 -> 11.71
+#   fp32 SGD               4.52 -> 4.44  12.00 -> 11.98       5.80 -> 5.83   20.25 -> 20.26
+#   MPT                    4.61 -> 4.59  12.06 -> 12.08       6.08 -> 6.05   20.15 -> 20.14
+#   AFP                    8.42 -> 8.37  13.45 -> 13.40       9.64 -> 9.65   21.72 -> 21.70
+#   MuPPET                10.22 -> 10.30 16.97 -> 16.82      11.34 -> 11.32  23.60 -> 23.53
+# MASCOT's mixed epochs of 250M ratings are level.  fp32 SGD at k = 128 stores through row windows, has no choice of stores to
+# gain from, and loses 0.6 to 1 % from 400k to 30M ratings: its file goes without them.
+UNIFORM_BRANCH_FLAGS = ["-mllvm", "-structurizecfg-skip-uniform-regions=true", "-mllvm", "-enable-tail-merge=false"]
+STRUCTURISED = {"launch_sgd_k128.hip"}
+EXTRA_FLAGS = os.environ.get("MF_HIPCC_FLAGS", "").split()
+KERNEL_SOURCES = ["launch_mascot_plain.hip", "launch_mascot_sampled.hip", "launch_mascot_binary16.hip", "launch_muppet.hip", "launch_afp.hip", "hogwild_launch.hip", "launch_sgd_k128.hip",
+                  "launch_mem_quant.hip", "aux_kernels.hip", "sort_shuffle.hip", "launch_mascot.hip"]
 HOST_SOURCES = ["train.cpp"]
 CLI_SOURCES = ["main.cpp", "io_utils.cpp"]
 EVAL_SOURCES = ["test_mf_main.cpp", "io_utils.cpp"]
@@ -51,7 +63,7 @@ def _run(cmd):
 
 def device_flags(src):
     """The compiler flags of one .hip file."""
-    return DEVICE_FLAGS
+    return DEVICE_FLAGS + ([] if src in STRUCTURISED else UNIFORM_BRANCH_FLAGS) + EXTRA_FLAGS
 
 
 def flags_record():

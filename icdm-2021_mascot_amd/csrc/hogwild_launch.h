@@ -196,25 +196,26 @@ static int launch_hot(const char* who, const Call& c, const typename Rule::Param
     return MF_OK;
 }
 
-// Instantiates Rule<K, COH> for the four (k, coherence) combinations; P is the parameter pack type,
-// identical across instantiations apart from the template arguments.
+// Instantiates Rule<K, COH> for both coherences; make fills the parameter pack, whose type is identical across instantiations
+// apart from the template arguments.
+template <int K, template <int, bool> class Rule, class MakeParams>
+static int launch_coh(const char* who, const Call& c, MakeParams make, size_t lds, void* stream, Range r)
+{
+    if (c.coherent) { auto a = make(typename Rule<K, true>::Params{}); return launch<Rule<K, true>>(who, c, a, lds, stream, r); }
+    auto a = make(typename Rule<K, false>::Params{}); return launch<Rule<K, false>>(who, c, a, lds, stream, r);
+}
 template <template <int, bool> class Rule, class MakeParams>
 static int launch_k_coh(const char* who, int k, const Call& c, MakeParams make, size_t lds, void* stream, Range r)
 {
-    if (k == 128) {
-        if (c.coherent) { auto a = make(typename Rule<128, true>::Params{}); return launch<Rule<128, true>>(who, c, a, lds, stream, r); }
-        auto a = make(typename Rule<128, false>::Params{}); return launch<Rule<128, false>>(who, c, a, lds, stream, r);
-    }
-    if (c.coherent) { auto a = make(typename Rule<64, true>::Params{}); return launch<Rule<64, true>>(who, c, a, lds, stream, r); }
-    auto a = make(typename Rule<64, false>::Params{}); return launch<Rule<64, false>>(who, c, a, lds, stream, r);
+    return k == 128 ? launch_coh<128, Rule>(who, c, make, lds, stream, r) : launch_coh<64, Rule>(who, c, make, lds, stream, r);
 }
 // Updates in flight during a launch of num_workers workers of Rule at this k (the build with the hot-row code and
 // coherent stores, which is what a run with hot-row tables launches): resident wavefronts x ratings per wavefront.
-template <template <int, bool> class Rule>
-static float inflight_updates(int k, uint32_t num_workers, size_t lds, uint32_t resident_cap)
+template <class Rule>
+static float inflight_of(uint32_t num_workers, size_t lds, uint32_t resident_cap)
 {
     int blocks = 0, dev = 0, cus = 0;
-    const void* kernel = k == 128 ? reinterpret_cast<const void*>(&hogwild_kernel<Rule<128, true>, true>) : reinterpret_cast<const void*>(&hogwild_kernel<Rule<64, true>, true>);
+    const void* kernel = reinterpret_cast<const void*>(&hogwild_kernel<Rule, true>);
     // a launch held to resident_cap workers runs with the LDS size that does the holding
     if (const size_t padded = lds_for_resident_cap(kernel, lds, resident_cap, num_workers)) lds = padded;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, kBlock, lds);
@@ -223,11 +224,17 @@ static float inflight_updates(int k, uint32_t num_workers, size_t lds, uint32_t 
         return 0.f;
     }
     const double resident = (double)blocks * kWavesPerBlock * cus;
-    const double ahead = k == 128 ? Rule<128, true>::kAhead + 1 : Rule<64, true>::kAhead + 1;
+    const double ahead = Rule::kAhead + 1;
     return (float)(((double)num_workers < resident ? (double)num_workers : resident) * ahead);
+}
+template <template <int, bool> class Rule>
+static float inflight_updates(int k, uint32_t num_workers, size_t lds, uint32_t resident_cap)
+{
+    return k == 128 ? inflight_of<Rule<128, true>>(num_workers, lds, resident_cap) : inflight_of<Rule<64, true>>(num_workers, lds, resident_cap);
 }
 // cap: mf_hogwild_options::resident_workers of the launch (0 = none)
 float inflight_sgd(int k, uint32_t num_workers, uint32_t cap);          // hogwild_launch.hip
+float inflight_sgd_k128(uint32_t num_workers, uint32_t cap);            // launch_sgd_k128.hip
 float inflight_mpt(int k, uint32_t num_workers, uint32_t cap);
 float inflight_mem_quant(int k, uint32_t num_workers, uint32_t cap);    // launch_mem_quant.hip
 float inflight_muppet(int k, uint32_t num_workers, uint32_t cap);       // launch_muppet.hip
@@ -235,5 +242,7 @@ float inflight_afp(int k, uint32_t num_workers, uint32_t cap);          // launc
 float inflight_mascot(int k, uint32_t num_workers, uint32_t user_groups, uint32_t item_groups, uint32_t cap);   // launch_mascot_binary16.hip
 
 static Range whole_epoch(const Call& c) { Range r; r.begin = 0; r.end = c.s.range_end; return r; }
+// fp32 SGD at k = 128 (launch_sgd_k128.hip)
+int launch_sgd_k128(const char* who, const Call& c, float* p, float* q, float lrate, float lambda, void* stream);
 
 }  // namespace mf

@@ -1,5 +1,5 @@
 // extern "C" launchers of the Hogwild update kernels: process-wide settings, closed forms of the schedule, and the
-// fp32 SGD and MPT entry points (the other rules' entry points sit in launch_*.hip).
+// fp32 SGD and MPT entry points (the other rules' entry points, and fp32 SGD's kernels at k = 128, sit in launch_*.hip).
 #include "hogwild_launch.h"
 #include "rules_fp32.h"
 
@@ -88,7 +88,7 @@ int replica_sync(const ReplicaSide& user, const ReplicaSide& item, int k, bool m
     return launch_status("replica_sync");
 }
 
-float inflight_sgd(int k, uint32_t num_workers, uint32_t cap) { return inflight_updates<SgdRule>(k, num_workers, 0, cap); }
+float inflight_sgd(int k, uint32_t num_workers, uint32_t cap) { return k == 128 ? inflight_sgd_k128(num_workers, cap) : inflight_of<SgdRule<64, true>>(num_workers, 0, cap); }
 float inflight_mpt(int k, uint32_t num_workers, uint32_t cap) { return inflight_updates<MptRule>(k, num_workers, 0, cap); }
 
 }  // namespace mf
@@ -165,7 +165,8 @@ int mf_single_sgd_hogwild_opt(const mf_node* R, uint32_t nnz, float* p, float* q
     if (int rc = check_schedule("mf_single_sgd_hogwild", R, nnz, k, num_workers, update_count, update_vector_size, options)) return rc;
     if (!p || !q) return invalid("mf_single_sgd_hogwild: null model pointer");
     const Call c = make_call(R, nnz, num_workers, update_count, update_vector_size, seed, epoch, window_start, options);
-    return launch_k_coh<SgdRule>("mf_single_sgd_hogwild", k, c, [&](auto a) { a.p = p; a.q = q; a.lrate = lrate; a.lambda = lambda; return a; }, 0, stream, whole_epoch(c));
+    if (k == 128) return launch_sgd_k128("mf_single_sgd_hogwild", c, p, q, lrate, lambda, stream);
+    return launch_coh<64, SgdRule>("mf_single_sgd_hogwild", c, [&](auto a) { a.p = p; a.q = q; a.lrate = lrate; a.lambda = lambda; return a; }, 0, stream, whole_epoch(c));
 }
 int mf_single_sgd_hogwild(const mf_node* R, uint32_t nnz, float* p, float* q, int k,
                           uint32_t num_workers, uint32_t update_count, uint32_t update_vector_size,

@@ -29,5 +29,7 @@ def test_the_build_records_every_files_flags(tmp_path, monkeypatch):
     assert sorted(lines) == sorted(builder.KERNEL_SOURCES)
     for src, flags in lines.items():
         assert flags.split() == builder.device_flags(src)
-    monkeypatch.setattr(builder, "DEVICE_FLAGS", builder.DEVICE_FLAGS + ["-DX=1"])
+    assert builder.STRUCTURISED < set(lines)
+    assert {src for src, flags in lines.items() if builder.UNIFORM_BRANCH_FLAGS[1] not in flags} == builder.STRUCTURISED
+    monkeypatch.setattr(builder, "EXTRA_FLAGS", ["-DX=1"])
     assert all(line.endswith(" -DX=1") for line in builder.flags_record().splitlines())
