@@ -461,31 +461,46 @@ __global__ __launch_bounds__(kStreamBlock) void iota_kernel(uint32_t* __restrict
     const uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) a[i] = i;
 }
-// user_item_histogram (preprocess_utils.h:13-19).  A workgroup counts one range of ids in its LDS, over one chunk of the
-// ratings: global atomics on scattered counters go to the memory side one by one, and with Zipf-like popularity a few
-// counters would take percents of them.  User and item ids are laid end to end and cut into ranges of kHistBins; the
-// workgroups of one chunk sit on one XCD, so that its L2 hands them the same ratings.  How far the ids reach is not
-// an argument: every workgroup takes the largest ids of the same kHistSample ratings, spread over the input, and the few
-// above them are added in memory by the workgroups of the first and the last range.
-// Ids that reach further than kHistRanges ranges are counted in a hash table in LDS instead, kHistSlots (id, count) slots per
-// side, a slot claimed by the first id that hashes to it (two probes); ids that find both taken go to memory.  At
-// 100M ratings the ranges take 1.5 ms for 15 of them whatever the popularity is, and from 17 on, with one chunk per XCD, they would take 3; the table takes 3.3 ms for 250M ratings of 1M + 625k ids under Zipf(1.2), where nearly all ids find a slot,
-// 6.1 for 100M under Zipf(0.8) (tables half as large, in smaller workgroups: 4.1 and 6.9).
-// What bounds it is the L1 and the instructions per id: each range's workgroup reads the whole chunk.  100M ratings over 480k + 17.8k ids: 0.84 ms
-// (0.97 with every result looked at by itself, 1.63 without the next tile's loads in flight); with a 4096-entry hash table per
-// side and workgroup, which sends two thirds of the user counts to memory, about 4.2.
+// user_item_histogram (preprocess_utils.h:13-19).  Global atomics on scattered counters go to the memory side one by one, and with
+// Zipf-like popularity a few counters would take percents of them, so ids are counted in LDS first.  Three ways:
+//   few     up to kHistFew ratings: a workgroup counts its ratings in a hash table, kHistFewLog bits of (id, count) slots per side, a
+//           slot claimed by the first id that hashes to it (two probes); ids that find both taken go to memory, and the table
+//           follows at the end.
+//   ranges  a workgroup counts one range of ids, over one chunk of the ratings.  User and item ids are laid end to end and cut
+//           into ranges of kHistBins; the workgroups of one chunk sit on one XCD, so that its L2 hands them the same ratings.  How
+//           far the ids reach is not an argument: every workgroup takes the largest ids of the same kHistSample ratings, spread over
+//           the input, and the few above them are added in memory by the workgroups of the first and the last range.
+//   hashed  as few, with tables twice as large on one workgroup per compute unit: ids that reach past kHistRanges ranges, or past
+//           kHistSure while few different ones make up most of the ratings (or there are less than kHistSampled ratings).
+// What bounds the ranges is a workgroup's pass over its chunk (L1 and the instructions per id), so their time follows
+// ratings / chunks: 100M ratings take 0.46 ms in 3 ranges, 0.81 in 7 (1.63 without the next tile's loads in flight), 1.55 in 15,
+// 2.95 from 17 to 32, up to a fifth more under Zipf(1.2).  A workgroup with ids of both sides makes two passes and the others wait
+// for it: 50M ratings of 1M + 200k ids took 1.67 ms in 15 ranges with one such and take 0.81 in 16 without.  In front of that come
+// 13 to 20 us: 160 KB of counters cleared, the sample, the counters' way to memory.
+// The tables' time follows the ids that find no slot.  50M ratings of 1M + 625k ids (21 ranges), hashed / ranges: flat 3.69 / 1.54 ms,
+// Zipf(0.8) 3.10 / 1.54, Zipf(1.0) 1.79 / 1.53, Zipf(1.1) 1.12 / 1.54, Zipf(1.2) 0.68 / 1.54.  The sample tells them apart: 7942, 6980, 4653, 3441
+// and 2341 different hash values of both sides, and the line is at kHistDistinct.  With few ratings the tables are the faster way
+// for flat ids, too: 39 / 49 us at 400k, 54 / 49 at 600k.
+// Up to kHistFew ratings the same goes for fewer ids: 100k ratings of 480k + 17.8k ids take 14 us (flat) and 8 (Zipf(1.2)), where the
+// ranges took 27, one rating 4 instead of 14 to 21.  At 200k ratings the tables' lead is 18 to 21 against 22 us there, but with up
+// to 5k ids, where all tables add to the same few counters, they take 38 to 56 against 13 to 16.  For the sake of these the
+// workgroups are few, too: with 128 instead of kHistFewGrid 100k ratings of 1000 + 500 ids took 29 us instead of 13, at 1 to 3 us
+// less where there are many ids.
 //
-// Counters are 16 bits wide, twice as many ids per range.  The thread that brings one to 2^15 moves 2^15 to memory; it has done
+// Counters of a range are 16 bits wide, twice as many ids per range.  The thread that brings one to 2^15 moves 2^15 to memory; it has done
 // so before the next barrier, and between two barriers there are kHistBlock * kHistUnroll = 2^14 ids per side at most.
 constexpr int kHistBlock = 1024;
 constexpr uint32_t kHistUnroll = 16;
 constexpr uint32_t kHistHalf = 40448, kHistBins = 2 * kHistHalf;      // words, each the counters of ids x and x + kHistHalf of the range
-constexpr uint32_t kHistRanges = 16, kHistGrid = 256;                 // one workgroup per compute unit, 32 per XCD
-constexpr uint32_t kHistLog = 13, kHistSlots = 1u << kHistLog;
-constexpr uint32_t kHistSample = 4 * kHistBlock;
-constexpr uint32_t kHistChunkMin = 1u << 14;                          // ratings: below, emptying the counters costs more than counting
+constexpr uint32_t kHistGrid = 256, kHistPerXcd = kHistGrid / kXcds;  // one workgroup per compute unit
+constexpr uint32_t kHistRanges = kHistPerXcd, kHistSure = 16, kHistDistinct = 4000;
+constexpr uint32_t kHistSampled = 1u << 19;
+constexpr uint32_t kHistLog = 13, kHistSlots = 1u << kHistLog, kHistHashedMin = 4096;      // ratings of a workgroup
+constexpr uint32_t kHistFew = 1u << 17, kHistFewLog = 12, kHistFewGrid = 32;
+constexpr uint32_t kHistSample = 4 * kHistBlock, kHistSeenBits = 16;
+constexpr uint32_t kHistChunkMin = 1u << 14;                          // ratings
 constexpr size_t kHistLds = (size_t)kHistHalf * 4;
-static_assert(4 * kHistSlots <= kHistHalf, "the hash tables fit where the counters are");
+static_assert(4 * kHistSlots <= kHistHalf && (2u << kHistSeenBits) / 32 <= kHistHalf, "the hash tables and the sample's bits fit where the counters are");
 static_assert(kHistBlock * kHistUnroll + 0x8000u < 0x10000u, "a 16-bit counter cannot overflow between two barriers");
 struct HistogramRange {
     uint32_t* bin;            // LDS
@@ -525,9 +540,9 @@ struct HistogramRange {
         }
     }
 };
-__device__ __forceinline__ void hashed_count(uint32_t* tag, uint32_t* cnt, uint32_t id, uint32_t* global_bin)
+template <uint32_t LOG> __device__ __forceinline__ void hashed_count(uint32_t* tag, uint32_t* cnt, uint32_t id, uint32_t* global_bin)
 {
-    uint32_t s = (id * 2654435761u) >> (32 - kHistLog);
+    uint32_t s = (id * 2654435761u) >> (32 - LOG);
 #pragma unroll
     for (int probe = 0; probe < 2; ++probe, s ^= 1u) {
         uint32_t t = tag[s];
@@ -536,59 +551,94 @@ __device__ __forceinline__ void hashed_count(uint32_t* tag, uint32_t* cnt, uint3
     }
     atomicAdd(&global_bin[id], 1u);
 }
-// tab: 4 * kHistSlots words of LDS, zero
-__device__ __forceinline__ void histogram_hashed(const mf_node* __restrict__ R, uint32_t n, uint32_t* user_bin, uint32_t* item_bin, uint32_t* tab)
+// Ratings [begin, end), AHEAD of each lane in flight.  tab: 4 << LOG words of LDS, zero: user tags, user counts, item tags, item counts.
+template <uint32_t LOG, uint32_t AHEAD>
+__device__ __forceinline__ void histogram_hashed(const mf_node* __restrict__ R, uint64_t begin, uint64_t end, uint32_t* user_bin, uint32_t* item_bin, uint32_t* tab)
 {
-    uint32_t* utag = tab, *ucnt = tab + kHistSlots, *itag = tab + 2 * kHistSlots, *icnt = tab + 3 * kHistSlots;
-    const uint64_t begin = (uint64_t)n * blockIdx.x / kHistGrid, end = (uint64_t)n * (blockIdx.x + 1u) / kHistGrid;
-    constexpr uint32_t kAhead = 8;
-    for (uint64_t base = begin; base < end; base += kHistBlock * kAhead) {
+    uint32_t* utag = tab, *ucnt = tab + (1u << LOG), *itag = tab + (2u << LOG), *icnt = tab + (3u << LOG);
+    for (uint64_t base = begin; base < end; base += kHistBlock * AHEAD) {
         const uint32_t* w = reinterpret_cast<const uint32_t*>(R + base);
-        const uint32_t left = end - base < kHistBlock * kAhead ? (uint32_t)(end - base) : kHistBlock * kAhead;
-        uint32_t u[kAhead], v[kAhead];
+        const uint32_t left = end - base < kHistBlock * AHEAD ? (uint32_t)(end - base) : kHistBlock * AHEAD;
+        uint32_t u[AHEAD], v[AHEAD];
 #pragma unroll
-        for (uint32_t j = 0; j < kAhead; ++j) {
+        for (uint32_t j = 0; j < AHEAD; ++j) {
             const uint32_t o = min(j * kHistBlock + threadIdx.x, left - 1u) * 3u;
             u[j] = __builtin_nontemporal_load(w + o + 1u); v[j] = __builtin_nontemporal_load(w + o + 2u);
         }
 #pragma unroll
-        for (uint32_t j = 0; j < kAhead; ++j) {
+        for (uint32_t j = 0; j < AHEAD; ++j) {
             if (j * kHistBlock + threadIdx.x >= left) continue;
-            hashed_count(utag, ucnt, u[j], user_bin);
-            hashed_count(itag, icnt, v[j], item_bin);
+            hashed_count<LOG>(utag, ucnt, u[j], user_bin);
+            hashed_count<LOG>(itag, icnt, v[j], item_bin);
         }
     }
     __syncthreads();
-    for (uint32_t s = threadIdx.x; s < kHistSlots; s += kHistBlock) {
+    for (uint32_t s = threadIdx.x; s < (1u << LOG); s += kHistBlock) {
         if (utag[s]) atomicAdd(&user_bin[utag[s] - 1u], ucnt[s]);
         if (itag[s]) atomicAdd(&item_bin[itag[s] - 1u], icnt[s]);
     }
 }
+__global__ __launch_bounds__(kHistBlock) void histogram_few_kernel(const mf_node* __restrict__ R, uint32_t n, uint32_t per_block, uint32_t* user_bin, uint32_t* item_bin)
+{
+    __shared__ uint32_t tab[4u << kHistFewLog];
+    for (uint32_t i = threadIdx.x; i < 4u << kHistFewLog; i += kHistBlock) tab[i] = 0u;
+    __syncthreads();
+    const uint64_t begin = (uint64_t)blockIdx.x * per_block, end = begin + per_block;
+    histogram_hashed<kHistFewLog, 4>(R, begin, end < n ? end : n, user_bin, item_bin, tab);
+}
 __global__ __launch_bounds__(kHistBlock) void histogram_kernel(const mf_node* __restrict__ R, uint32_t n, uint32_t* user_bin, uint32_t* item_bin)
 {
     extern __shared__ uint32_t hist_bin[];
-    __shared__ uint32_t reach[2];
-    if (threadIdx.x < 2) reach[threadIdx.x] = 0u;
-    for (uint32_t i = threadIdx.x; i < kHistHalf; i += kHistBlock) hist_bin[i] = 0u;
-    __syncthreads();
-    uint32_t mu = 0, mv = 0;
+    __shared__ uint32_t reach[2], distinct;
+    uint32_t su[kHistSample / kHistBlock], sv[kHistSample / kHistBlock];
 #pragma unroll
     for (uint32_t j = 0; j < kHistSample / kHistBlock; ++j) {
         const uint32_t at = (uint32_t)((uint64_t)n * (j * kHistBlock + threadIdx.x) / kHistSample);
-        mu = max(mu, R[at].u); mv = max(mv, R[at].i);
+        su[j] = R[at].u; sv[j] = R[at].i;
     }
-    atomicMax(&reach[0], mu); atomicMax(&reach[1], mv);
+    if (threadIdx.x < 2) reach[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) distinct = 0u;
+    for (uint32_t i = threadIdx.x; i < kHistHalf; i += kHistBlock) hist_bin[i] = 0u;      // while the sample is on its way
+    __syncthreads();
+    uint32_t mu = 0, mv = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kHistSample / kHistBlock; ++j) { mu = max(mu, su[j]); mv = max(mv, sv[j]); }
+    for (int d = kWave / 2; d; d >>= 1) { mu = max(mu, (uint32_t)__shfl_xor((int)mu, d)); mv = max(mv, (uint32_t)__shfl_xor((int)mv, d)); }
+    if ((threadIdx.x & 63u) == 0u) { atomicMax(&reach[0], mu); atomicMax(&reach[1], mv); }
     __syncthreads();
     const uint32_t most = (kHistRanges + 1u) * kHistBins;
     const uint32_t users = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(reach[0], most - 1u)) + 1u;
     const uint32_t items = (uint32_t)__builtin_amdgcn_readfirstlane((int)min(reach[1], most - 1u)) + 1u;
-    // the items begin a range of their own where that takes no more ranges: then no workgroup reads both ids
     const uint32_t user_ranges = (users + kHistBins - 1u) / kHistBins, apart = user_ranges + (items + kHistBins - 1u) / kHistBins;
-    const uint32_t ranges = (users + items + kHistBins - 1u) / kHistBins;
-    if (ranges > kHistRanges) { histogram_hashed(R, n, user_bin, item_bin, hist_bin); return; }
-    const uint32_t item_base = apart == ranges ? user_ranges * kHistBins : users;
+    const uint32_t together = (users + items + kHistBins - 1u) / kHistBins;
+    bool hashed = together > kHistRanges || (together > kHistSure && n < kHistSampled);
+    if (!hashed && together > kHistSure) {
+        // how many different ids the sample has: a bit per side and hash value, counted and cleared
+        constexpr uint32_t kWords = (1u << kHistSeenBits) / 32;
+#pragma unroll
+        for (uint32_t j = 0; j < kHistSample / kHistBlock; ++j) {
+            const uint32_t hu = (su[j] * 2654435761u) >> (32 - kHistSeenBits), hv = (sv[j] * 2654435761u) >> (32 - kHistSeenBits);
+            atomicOr(&hist_bin[hu / 32u], 1u << (hu % 32u));
+            atomicOr(&hist_bin[kWords + hv / 32u], 1u << (hv % 32u));
+        }
+        __syncthreads();
+        uint32_t count = 0;
+        for (uint32_t i = threadIdx.x; i < 2u * kWords; i += kHistBlock) { count += (uint32_t)__popc(hist_bin[i]); hist_bin[i] = 0u; }
+        for (int d = kWave / 2; d; d >>= 1) count += (uint32_t)__shfl_xor((int)count, d);
+        if ((threadIdx.x & 63u) == 0u) atomicAdd(&distinct, count);
+        __syncthreads();
+        hashed = distinct < kHistDistinct;
+    }
+    if (hashed) {
+        const uint32_t blocks = min(kHistGrid, n / kHistHashedMin + 1u);
+        if (blockIdx.x < blocks) histogram_hashed<kHistLog, 8>(R, (uint64_t)n * blockIdx.x / blocks, (uint64_t)n * (blockIdx.x + 1u) / blocks, user_bin, item_bin, hist_bin);
+        return;
+    }
+    // The items begin a range of their own unless the one more range takes half of the chunks
+    const bool split = apart == together || (apart <= kHistPerXcd && 2u * (kHistPerXcd / apart) > kHistPerXcd / together);
+    const uint32_t ranges = split ? apart : together, item_base = split ? user_ranges * kHistBins : users;
     const uint32_t xcd = blockIdx.x % kXcds, local = blockIdx.x / kXcds;
-    const uint32_t per_xcd = kHistGrid / kXcds / ranges, by_size = n / kHistChunkMin + 1u;
+    const uint32_t per_xcd = kHistPerXcd / ranges, by_size = n / kHistChunkMin + 1u;
     const uint32_t chunks = min(per_xcd * kXcds, by_size), chunk = xcd + kXcds * (local / ranges);
     if (local / ranges >= per_xcd || chunk >= chunks) return;
     const uint32_t first = local % ranges * kHistBins, last = first + kHistBins;
@@ -850,6 +900,11 @@ int mf_user_item_histogram(const mf_node* R, uint32_t n, uint32_t* user_bin, uin
 {
     if (n == 0) return MF_OK;
     if (!R || !user_bin || !item_bin) return invalid("mf_user_item_histogram: null pointer");
+    if (n <= kHistFew) {
+        const uint32_t share = (n + kHistFewGrid - 1) / kHistFewGrid, per_block = share < (uint32_t)kHistBlock ? (uint32_t)kHistBlock : share;
+        hipLaunchKernelGGL(histogram_few_kernel, dim3((n + per_block - 1) / per_block), dim3(kHistBlock), 0, as_stream(stream), R, n, per_block, user_bin, item_bin);
+        return launch_status("mf_user_item_histogram");
+    }
     if (int rc = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(histogram_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kHistLds),
                            "hipFuncSetAttribute(MaxDynamicSharedMemorySize)")) return rc;
     hipLaunchKernelGGL(histogram_kernel, dim3(kHistGrid), dim3(kHistBlock), kHistLds, as_stream(stream), R, n, user_bin, item_bin);

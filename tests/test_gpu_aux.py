@@ -422,8 +422,7 @@ def test_workspace_forms_equal_the_allocating_forms(orc):
             h.mf_synth_build_tables(C.addressof(c), 9, tables.data_ptr(), need - 1, st)
 
 
-# ids in one range of the counting kernel (80896), across two, in the item ranges behind the users', in 15 ranges, in too many for it, and
-# counters that pass 2^15 several times
+# up to 131072 ratings a table per workgroup; above, ids in several ranges of 80896 and (the last two of more than a million ids) in too many
 @pytest.mark.parametrize("n,n_users,n_items,hot", [(1, 1, 1, False), (63, 80895, 1, False), (16385, 80896, 80897, False), (70_001, 3, 90_000, True),
                                                    (300_007, 161_793, 161_000, True), (900_001, 3_000_000, 700_000, True), (500_001, 1_000_000, 200_000, True), (400_003, 10, 5_000_000, False)])
 def test_histogram_reindex_ranges(n, n_users, n_items, hot):
@@ -447,6 +446,28 @@ def test_histogram_reindex_ranges(n, n_users, n_items, hot):
     assert np.array_equal(ib.cpu().numpy(), np.bincount(R["i"], minlength=n_items))
     got = from_dev(dR, mfutil.NODE)
     assert np.array_equal(got["r"], R["r"]) and np.array_equal(got["u"], u2s[R["u"]]) and np.array_equal(got["i"], i2s[R["i"]])
+
+
+# Both sides of every line of the choice: table or ranges by the number of ratings; 21 and 32 ranges of which few ids make up most
+# of the ratings or not; one range too many; users and items sharing a range (1 and 16 ranges) or not (2 and 17).
+@pytest.mark.parametrize("n,n_users,n_items,share", [(131072, 480_000, 17_800, 0.0), (131073, 480_000, 17_800, 0.0), (131073, 480_000, 17_800, 0.9),
+                                                     (524_287, 1_000_000, 625_000, 0.0), (524_288, 1_000_000, 625_000, 0.0), (524_288, 1_000_000, 625_000, 0.9), (600_001, 2_500_000, 80_896, 0.0),
+                                                     (600_001, 2_500_000, 80_896, 0.9), (600_001, 2_588_672, 80_896, 0.0), (140_001, 70_000, 10_700, 0.3),
+                                                     (140_001, 80_896, 10_700, 0.3), (140_001, 1_250_000, 44_000, 0.3), (600_001, 1_200_000, 161_000, 0.3)])
+def test_histogram_choice(n, n_users, n_items, share):
+    import torch
+    h = mfutil.hip()
+    g = torch.Generator(device="cuda").manual_seed(n + n_users)
+    R = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+    for word, ids in ((1, n_users), (2, n_items)):
+        R[:, word] = torch.randint(0, ids, (n,), generator=g, device="cuda")
+        popular = torch.rand(n, generator=g, device="cuda") < share
+        R[:, word][popular] = torch.randint(ids - min(ids, 100), ids, (n,), generator=g, device="cuda", dtype=torch.int32)[popular]
+        R[0, word] = ids - 1            # among the sampled ratings: the reach is known
+    ub, ib = torch.full((n_users,), 7, dtype=torch.int32, device="cuda"), torch.zeros(n_items, dtype=torch.int32, device="cuda")
+    h.mf_user_item_histogram(R.data_ptr(), n, ub.data_ptr(), ib.data_ptr(), mfutil.stream_ptr())
+    assert torch.equal(ub.long(), torch.bincount(R[:, 1], minlength=n_users) + 7)
+    assert torch.equal(ib.long(), torch.bincount(R[:, 2], minlength=n_items))
 
 
 # remainders of 64 ratings and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
