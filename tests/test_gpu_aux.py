@@ -470,6 +470,28 @@ def test_histogram_choice(n, n_users, n_items, share):
     assert torch.equal(ib.long(), torch.bincount(R[:, 2], minlength=n_items))
 
 
+# A range's counters are 16 bits wide, ids x and x + 40448 of a range in one word: ids that pass 2^15 at least twice in every chunk of the
+# ratings, in either half of a word, of users, of items, and of items that share a range with users
+@pytest.mark.parametrize("n,chunks,n_users,n_items,user,item", [(3_000_001, 16, 1_000_000, 200_000, 5 * 80896 + 100, 80896 + 17),
+                                                                (3_000_001, 16, 1_000_000, 200_000, 5 * 80896 + 40448 + 7, 80896 + 50_000),
+                                                                (3_000_001, 16, 1_000_000, 200_000, 999_999, 199_999),
+                                                                (25_000_003, 256, 70_000, 10_700, 5, 10_699), (25_000_003, 256, 70_000, 10_700, 69_999, 0)])
+def test_histogram_counters_move_to_memory(n, chunks, n_users, n_items, user, item):
+    import torch
+    h = mfutil.hip()
+    g = torch.Generator(device="cuda").manual_seed(n + user)
+    R = torch.zeros((n, 3), dtype=torch.int32, device="cuda")
+    for word, ids, hot in ((1, n_users, user), (2, n_items, item)):
+        R[:, word] = torch.randint(0, ids, (n,), generator=g, device="cuda")
+        R[:, word][torch.rand(n, generator=g, device="cuda") < 0.8] = hot
+        per_chunk = (R[:, word] == hot).long().cumsum(0)[[n * (c + 1) // chunks - 1 for c in range(chunks)]].diff()
+        assert int(per_chunk.min()) > 2 << 15
+    ub, ib = torch.zeros(n_users, dtype=torch.int32, device="cuda"), torch.zeros(n_items, dtype=torch.int32, device="cuda")
+    h.mf_user_item_histogram(R.data_ptr(), n, ub.data_ptr(), ib.data_ptr(), mfutil.stream_ptr())
+    assert torch.equal(ub.long(), torch.bincount(R[:, 1], minlength=n_users))
+    assert torch.equal(ib.long(), torch.bincount(R[:, 2], minlength=n_items))
+
+
 # remainders of 64 ratings and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
 # ratings of ids in no group; the sums in binary64 on the host from the same rows (a binary32 dot of k products is off by k / 2^24
 # of the sum of their sizes at most)
