@@ -679,24 +679,27 @@ __global__ __launch_bounds__(kHistBlock) void histogram_kernel(const mf_node* __
 // The ratings as a stream of words, four per lane and load: word w is a rating value, a user or an item by w % 3 (for the
 // words of the t-th four: (t + j) % 3), and the values go back with the ids around them, so that whole lines are read and written.
 // What bounds it is the lookups, a line each.  With a thread per rating, two strided loads and two strided stores, 100M ratings
-// took 1.15 ms; this takes 0.95, 200M lookups that fetch 13 TB/s of lines from the L2.
+// took 1.25 ms; this takes 1.05, 200M lookups that fetch 12 TB/s of lines from the L2.
+// UNROLL: fours of a lane whose lookups are in flight together.  While the lanes are few, more of them are better than more lookups
+// per lane: one against four, 100k ratings of 5M + 1M ids take 5 us instead of 7, 800k of 480k + 17.8k ids 7.9 instead of 8.7, 1.3M 12.4
+// instead of 11.9.
 typedef uint32_t Word4 __attribute__((ext_vector_type(4)));
 typedef Word4 Word4A4 __attribute__((aligned(4)));
-constexpr uint32_t kReindexUnroll = 4;
+template <uint32_t UNROLL>
 __global__ __launch_bounds__(kStreamBlock, 8) void reindex_kernel(uint32_t* R, const uint32_t* __restrict__ user2sorted, const uint32_t* __restrict__ item2sorted, uint64_t words)
 {
-    const uint64_t fours = words / 4, stride = (uint64_t)gridDim.x * kStreamBlock * kReindexUnroll;
+    const uint64_t fours = words / 4, stride = (uint64_t)gridDim.x * kStreamBlock * UNROLL;
     Word4A4* to = reinterpret_cast<Word4A4*>(R);
-    for (uint64_t base = (uint64_t)blockIdx.x * kStreamBlock * kReindexUnroll + threadIdx.x; base < fours; base += stride) {
-        Word4 x[kReindexUnroll], y[kReindexUnroll];
+    for (uint64_t base = (uint64_t)blockIdx.x * kStreamBlock * UNROLL + threadIdx.x; base < fours; base += stride) {
+        Word4 x[UNROLL], y[UNROLL];
 #pragma unroll
-        for (uint32_t i = 0; i < kReindexUnroll; ++i) {
+        for (uint32_t i = 0; i < UNROLL; ++i) {
             x[i] = Word4{0u, 0u, 0u, 0u};
             if (base + i * kStreamBlock < fours) x[i] = __builtin_nontemporal_load(to + base + i * kStreamBlock);
         }
         // no branches, which would wait for one lookup before the next: a lane with nothing to look up reads entry 0
 #pragma unroll
-        for (uint32_t i = 0; i < kReindexUnroll; ++i) {
+        for (uint32_t i = 0; i < UNROLL; ++i) {
             const uint64_t t = base + i * kStreamBlock;
             const uint32_t kind = (uint32_t)(t % 3u);
 #pragma unroll
@@ -707,7 +710,7 @@ __global__ __launch_bounds__(kStreamBlock, 8) void reindex_kernel(uint32_t* R, c
             }
         }
 #pragma unroll
-        for (uint32_t i = 0; i < kReindexUnroll; ++i)
+        for (uint32_t i = 0; i < UNROLL; ++i)
             if (base + i * kStreamBlock < fours) __builtin_nontemporal_store(y[i], to + base + i * kStreamBlock);
     }
     const uint64_t w = fours * 4 + threadIdx.x;      // up to three words are left
@@ -916,7 +919,11 @@ int mf_matrix_reconst_triplet(mf_node* R, const uint32_t* user2sorted_idx, const
     if (n == 0) return MF_OK;
     if (!R || !user2sorted_idx || !item2sorted_idx) return invalid("mf_matrix_reconst_triplet: null pointer");
     const uint64_t words = (uint64_t)n * 3;
-    hipLaunchKernelGGL(reindex_kernel, dim3(stream_grid(words / 4 + 1, kReindexUnroll)), dim3(kStreamBlock), 0, as_stream(stream), reinterpret_cast<uint32_t*>(R), user2sorted_idx, item2sorted_idx, words);
+    auto launch = [&](auto kernel, int unroll) {
+        hipLaunchKernelGGL(kernel, dim3(stream_grid(words / 4 + 1, unroll)), dim3(kStreamBlock), 0, as_stream(stream), reinterpret_cast<uint32_t*>(R), user2sorted_idx, item2sorted_idx, words);
+    };
+    if (words / 4 <= 3u << 18) launch(reindex_kernel<1>, 1);
+    else launch(reindex_kernel<4>, 4);
     return launch_status("mf_matrix_reconst_triplet");
 }
 

@@ -448,6 +448,24 @@ def test_histogram_reindex_ranges(n, n_users, n_items, hot):
     assert np.array_equal(got["r"], R["r"]) and np.array_equal(got["u"], u2s[R["u"]]) and np.array_equal(got["i"], i2s[R["i"]])
 
 
+# up to 786432 fours of words one per lane, then four; with the remainders of a four on both sides, and several rounds per lane
+@pytest.mark.parametrize("n", [1_048_575, 1_048_576, 1_048_577, 1_048_578, 1_048_579, 22_369_622])
+def test_reindex_sizes(n):
+    import torch
+    h = mfutil.hip()
+    g = torch.Generator(device="cuda").manual_seed(n)
+    n_users, n_items = 300_007, 5_003
+    R = torch.randint(-2 ** 31, 2 ** 31 - 1, (n + 1, 3), generator=g, device="cuda", dtype=torch.int64).int()
+    for word, ids in ((1, n_users), (2, n_items)):
+        R[:, word] = torch.randint(0, ids, (n + 1,), generator=g, device="cuda")
+    before = R.clone()
+    to_user = torch.randperm(n_users, generator=g, device="cuda").int()
+    to_item = torch.randperm(n_items, generator=g, device="cuda").int()
+    h.mf_matrix_reconst_triplet(R.data_ptr(), to_user.data_ptr(), to_item.data_ptr(), n, mfutil.stream_ptr())
+    assert torch.equal(R[n], before[n]) and torch.equal(R[:n, 0], before[:n, 0])
+    assert torch.equal(R[:n, 1], to_user[before[:n, 1].long()]) and torch.equal(R[:n, 2], to_item[before[:n, 2].long()])
+
+
 # Both sides of every line of the choice: table or ranges by the number of ratings; 21 and 32 ranges of which few ids make up most
 # of the ratings or not; one range too many; users and items sharing a range (1 and 16 ranges) or not (2 and 17).
 @pytest.mark.parametrize("n,n_users,n_items,share", [(131072, 480_000, 17_800, 0.0), (131073, 480_000, 17_800, 0.0), (131073, 480_000, 17_800, 0.9),
