@@ -72,10 +72,10 @@ __device__ __forceinline__ Float4 to_singles(Word2 v)
 // ---- scatter into grouped binary16 storage (model_init.cu:30-83) ---------------------------------
 // A wavefront takes kRowsPerWave consecutive rows: their destinations are looked up by one lane each, then every load takes
 // 16 bytes per lane (two rows at k = 128, four at k = 64) and all of them are in flight together.  One row at a time, each
-// behind its own chain of lookups, 480k + 17.8k rows at
-// k = 128 took 66 us per side on average to scatter and 146 to gather; this takes 47 and 36.
+// behind its own chain of lookups, 480k + 17.8k rows at k = 128 took 66 us per side on average to scatter and 146 to gather; this
+// takes 47 and 36.
 constexpr uint32_t kRowsPerWave = 16;
-static inline uint32_t rows_grid(uint32_t rows) { return stream_grid((uint64_t)rows * (kWave / kRowsPerWave)); }
+static inline uint32_t rows_grid(uint32_t rows, uint32_t per_wave = kRowsPerWave) { return stream_grid((uint64_t)rows * (kWave / per_wave)); }
 template <int K>
 __global__ __launch_bounds__(kBlock) void scatter_to_groups_kernel(const float* __restrict__ params, void* const* __restrict__ group_ptr,
                                                                   const uint32_t* __restrict__ group_end, const uint32_t* __restrict__ entity2group,
@@ -109,18 +109,21 @@ __global__ __launch_bounds__(kBlock) void scatter_to_groups_kernel(const float* 
 
 // ---- gather grouped storage into a dense fp32 matrix in sorted row order (mf_methods.cu:249-313) --
 // Rows and lanes as in the scatter.  A lane reads 8 bytes, which is all of a binary16 row, and where there are binary32 rows
-// among the wavefront's the other 8 bytes of those.
-template <int K>
+// among the wavefront's the other 8 bytes of those.  Few rows of k = 128
+// are spread over more wavefronts, kRowsFew each: 5000 binary32 rows take 4.9 us instead of 5.8 with kRowsPerWave, 20001 5.5 instead of 7.3
+// (one row at a time: 4.9 and 7.8).  At k = 64 both take the same (10001 rows 4.2 and 4.1), and so they do at 100k rows.
+constexpr uint32_t kRowsFew = 4, kGatherFew = 24576;
+template <int K, uint32_t ROWS>
 __global__ __launch_bounds__(kBlock) void gather_from_groups_kernel(void* const* __restrict__ group_ptr, const uint32_t* __restrict__ group_end,
                                                                    const uint8_t* __restrict__ prec, float* __restrict__ dense, uint32_t n, uint32_t groups)
 {
-    constexpr uint32_t kLanes = K / 4, kStep = kWave / kLanes, kSteps = kRowsPerWave / kStep;
+    constexpr uint32_t kLanes = K / 4, kStep = kWave / kLanes, kSteps = ROWS / kStep;
     const uint32_t lane = threadIdx.x & 63u, sub = lane / kLanes, col = lane % kLanes;
-    const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock * kRowsPerWave;
-    for (uint64_t base = ((uint64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6)) * kRowsPerWave; base < n; base += stride) {
+    const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock * ROWS;
+    for (uint64_t base = ((uint64_t)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6)) * ROWS; base < n; base += stride) {
         uint64_t src = 0;      // null: the row is in no group
         uint32_t single = 0;
-        if (lane < kRowsPerWave && base + lane < n) {
+        if (lane < ROWS && base + lane < n) {
             const uint32_t row = (uint32_t)(base + lane), g = group_of(group_end, groups, row);
             if (row <= group_end[g]) {
                 const uint32_t local = g ? row - group_end[g - 1] - 1 : row;
@@ -837,9 +840,12 @@ int mf_grouped_params2dense(void* const* group_ptr, const uint32_t* group_end_id
     if (k != 64 && k != 128) return invalid("mf_grouped_params2dense: k must be 64 or 128 (got %d)", k);
     if (n == 0) return MF_OK;
     if (!group_ptr || !group_end_idx || !group_prec_info || !dense || group_num == 0) return invalid("mf_grouped_params2dense: null pointer or no groups");
-    const uint32_t grid = rows_grid(n);
-    if (k == 128) hipLaunchKernelGGL(gather_from_groups_kernel<128>, dim3(grid), dim3(kBlock), 0, as_stream(stream), group_ptr, group_end_idx, group_prec_info, dense, n, group_num);
-    else hipLaunchKernelGGL(gather_from_groups_kernel<64>, dim3(grid), dim3(kBlock), 0, as_stream(stream), group_ptr, group_end_idx, group_prec_info, dense, n, group_num);
+    auto launch = [&](auto kernel, uint32_t rows) {
+        hipLaunchKernelGGL(kernel, dim3(rows_grid(n, rows)), dim3(kBlock), 0, as_stream(stream), group_ptr, group_end_idx, group_prec_info, dense, n, group_num);
+    };
+    if (k == 64) launch(gather_from_groups_kernel<64, kRowsPerWave>, kRowsPerWave);
+    else if (n <= kGatherFew) launch(gather_from_groups_kernel<128, kRowsFew>, kRowsFew);
+    else launch(gather_from_groups_kernel<128, kRowsPerWave>, kRowsPerWave);
     return launch_status("mf_grouped_params2dense");
 }
 

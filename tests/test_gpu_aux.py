@@ -510,6 +510,28 @@ def test_histogram_counters_move_to_memory(n, chunks, n_users, n_items, user, it
     assert torch.equal(ib.long(), torch.bincount(R[:, 2], minlength=n_items))
 
 
+# four rows of k = 128 per wavefront up to 24576, sixteen above, with remainders; groups of both precisions, and rows behind the last group
+@pytest.mark.parametrize("k", [64, 128])
+@pytest.mark.parametrize("rows", [3, 24575, 24576, 24577, 24593])
+def test_gather_rows(k, rows):
+    import torch
+    h = mfutil.hip()
+    g = torch.Generator(device="cuda").manual_seed(rows + k)
+    end = sorted({min(rows - 1, x) for x in (0, 1, 6, 1000, 1001, 20_000, rows - 3, rows - 2)})      # the last row is in no group
+    dense = (torch.randn((rows, k), generator=g, device="cuda") * 0.3).half().float()
+    ptr, keep, first = [], [], 0
+    for i, last in enumerate(end):
+        part = dense[first:last + 1].half() if i % 2 else dense[first:last + 1].clone()
+        keep.append(part)
+        ptr.append(part.data_ptr())
+        first = last + 1
+    d_ptr, d_end = torch.tensor(ptr, dtype=torch.int64, device="cuda"), torch.tensor(end, dtype=torch.int32, device="cuda")
+    prec = torch.tensor([1 - i % 2 for i in range(len(end))], dtype=torch.uint8, device="cuda")
+    out = torch.full((rows + 1, k), 9.0, device="cuda")
+    h.mf_grouped_params2dense(d_ptr.data_ptr(), d_end.data_ptr(), prec.data_ptr(), out.data_ptr(), k, rows, len(end), mfutil.stream_ptr())
+    assert torch.equal(out[:end[-1] + 1], dense[:end[-1] + 1]) and bool((out[end[-1] + 1:] == 9.0).all())
+
+
 # remainders of 64 ratings and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
 # ratings of ids in no group; the sums in binary64 on the host from the same rows (a binary32 dot of k products is off by k / 2^24
 # of the sum of their sizes at most)
