@@ -272,9 +272,11 @@ template <int K, bool SINGLE> __device__ __forceinline__ void rmse_wave(TestRati
     const uint64_t p = bcast(my.p, some), q = bcast(my.q, some); const uint32_t f = bcast(my.flags, some);
     if (my.flags & 4u) { my.p = p; my.q = q; my.flags = f | 4u; }
     const uint32_t lane16 = threadIdx.x & 15u;
+    // up to four ratings lie in the first batch: one takes 4.7 us (grouped, k = 128) instead of 5.7
+    const int batches = valid & ~0x000f000f000f000full ? 4 : 1;
     // not unrolled: four batches' loads in flight at once would not fit the registers of 16 wavefronts per compute unit
 #pragma unroll 1
-    for (int batch = 0; batch < 4; ++batch) {
+    for (int batch = 0; batch < batches; ++batch) {
         rmse_four<K, SINGLE>(my, lane16, acc);
         my.r = row_ror<4>(my.r); my.flags = row_ror<4>(my.flags);
         my.p = row_ror64<4>(my.p); my.q = row_ror64<4>(my.q);

@@ -532,11 +532,11 @@ def test_gather_rows(k, rows):
     assert torch.equal(out[:end[-1] + 1], dense[:end[-1] + 1]) and bool((out[end[-1] + 1:] == 9.0).all())
 
 
-# remainders of 64 ratings and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
+# remainders of 64 ratings (and of a wavefront's four batches of 16) and of the 16 rows a wavefront moves, rows at odd alignments, both precisions in every combination,
 # ratings of ids in no group; the sums in binary64 on the host from the same rows (a binary32 dot of k products is off by k / 2^24
 # of the sum of their sizes at most)
 @pytest.mark.parametrize("k", [64, 128])
-@pytest.mark.parametrize("test_n", [1, 63, 64, 65, 16 * 64 + 17, 40_003])
+@pytest.mark.parametrize("test_n", [1, 4, 5, 13, 17, 37, 63, 64, 65, 16 * 64 + 17, 40_003])
 def test_rmse_gather_mixed_rows(k, test_n):
     import torch
     h = mfutil.hip()
