@@ -150,9 +150,9 @@ __global__ __launch_bounds__(kShufBlock) void shuffle_place_kernel(PassArgs a)
 }
 static size_t place_lds(int bits) { const size_t bins = (size_t)1 << bits; return (bins + (bins < (size_t)kShufBlock ? (size_t)kShufBlock : bins)) * 4; }
 
-// 16 wavefronts on a compute unit, each lane with 8 ratings in flight: one workgroup of 1024 threads (147 KB of LDS) up to
-// 256 digits, two of 512 above.  The larger tile writes runs twice as long, and with half as many workgroups the cache lines
-// that are partly written at any time fit in an XCD's L2.
+// Each lane has 8 ratings in flight.  Up to 256 digits one workgroup of 1024 threads (147 KB of LDS) on a compute unit, two of 512 up
+// to 512 digits (76 KB each), one of 512 from there on (from 805M ratings).  The larger tile writes runs twice as long, and with half as many
+// workgroups the cache lines that are partly written at any time fit in an XCD's L2.
 template <int BLOCK, bool MOVED> __global__ __launch_bounds__(BLOCK) void shuffle_partition_kernel(PassArgs a)
 {
     constexpr uint32_t kTile = BLOCK * kPerThread;
@@ -213,6 +213,8 @@ template <int BLOCK, bool MOVED> __global__ __launch_bounds__(BLOCK) void shuffl
 }
 constexpr int kLargeTileBits = 8;
 static size_t partition_lds(int bits) { const size_t tile = (bits <= kLargeTileBits ? 1024u : 512u) * kPerThread; return tile * 18 + ((size_t)8 << bits); }
+// of the kernel on the whole card: 256 compute units of 160 KB
+static uint32_t partition_resident(int bits) { return 256u * (uint32_t)((160u << 10) / (partition_lds(bits) + 1024 / kWave * 4)); }
 
 // One bucket in order: by the kSubBits bits of the key after the bucket's, in LDS (0.75 ratings per value on average), then by
 // the whole key among the ratings that share them.  64 KB of LDS: two workgroups per compute unit.
@@ -319,7 +321,7 @@ static ShufflePlan shuffle_plan(uint32_t n)
     // as many workgroups as are resident, and at least four tiles for each where the input has them
     auto chunks = [](int b, uint64_t ratings, uint32_t segs) {
         const uint64_t tile = (b <= kLargeTileBits ? 1024u : 512u) * kPerThread, by_size = (ratings + 4 * tile - 1) / (4 * tile);
-        const uint32_t most = (b <= kLargeTileBits ? 256u : 512u) / segs;
+        const uint32_t most = partition_resident(b) / segs;
         return by_size < 1 || most < 1 ? 1u : (by_size < most ? (uint32_t)by_size : most);
     };
     p.chunks1 = chunks(p.bits1, n, 1);

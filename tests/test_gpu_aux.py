@@ -153,10 +153,12 @@ def test_shuffle_sizes(orc, n):
         assert np.array_equal(from_dev(dOut, mfutil.NODE).view(np.uint8), orc.shuffle(seed, R).view(np.uint8))
 
 
-def test_shuffle_beyond_the_large_tiles():
+# 17, 18 and 19 bits of buckets of 3072 ratings: passes of 9 + 8, 9 + 9 and 10 + 9
+@pytest.mark.parametrize("n", [(3072 << 16) + 77, (3072 << 17) + 77, (3072 << 18) + 77])
+def test_shuffle_beyond_the_large_tiles(n):
     """From 2^16 buckets of 3072 ratings on a pass has more than 8 bits and takes smaller tiles; against torch's sort of the keys."""
     import torch
-    h, n, seed = mfutil.hip(), (3072 << 16) + 77, 9
+    h, seed = mfutil.hip(), 9
     R = torch.empty((n, 3), dtype=torch.int32, device="cuda")
     for word in range(3):
         R[:, word] = torch.arange(n, dtype=torch.int32, device="cuda") + word
