@@ -483,9 +483,9 @@ __global__ __launch_bounds__(kStreamBlock) void iota_kernel(uint32_t* __restrict
 // for it: 50M ratings of 1M + 200k ids took 1.67 ms in 15 ranges with one such and take 0.81 in 16 without.  In front of that come
 // 13 to 20 us: 160 KB of counters cleared, the sample, the counters' way to memory.
 // The tables' time follows the ids that find no slot.  50M ratings of 1M + 625k ids (21 ranges), hashed / ranges: flat 3.69 / 1.54 ms,
-// Zipf(0.8) 3.10 / 1.54, Zipf(1.0) 1.79 / 1.53, Zipf(1.1) 1.12 / 1.54, Zipf(1.2) 0.68 / 1.54.  The sample tells them apart: 7942, 6980, 4653, 3441
-// and 2341 different hash values of both sides, and the line is at kHistDistinct.  With few ratings the tables are the faster way
-// for flat ids, too: 39 / 49 us at 400k, 54 / 49 at 600k.
+// Zipf(0.8) 3.10 / 1.54, Zipf(1.0) 1.79 / 1.53, Zipf(1.1) 1.12 / 1.54, Zipf(1.2) 0.68 / 1.54.  The sample tells them apart: 7942, 6980,
+// 4653, 3441 and 2341 different hash values of both sides, and the line is at kHistDistinct.  With few ratings the tables are the
+// faster way for flat ids, too: 39 / 49 us at 400k, 54 / 49 at 600k.
 // Up to kHistFew ratings the same goes for fewer ids: 100k ratings of 480k + 17.8k ids take 14 us (flat) and 8 (Zipf(1.2)), where the
 // ranges took 27, one rating 4 instead of 14 to 21.  At 200k ratings the tables' lead is 18 to 21 against 22 us there, but with up
 // to 5k ids, where all tables add to the same few counters, they take 38 to 56 against 13 to 16.  For the sake of these the
