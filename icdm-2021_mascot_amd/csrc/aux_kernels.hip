@@ -480,8 +480,9 @@ __global__ __launch_bounds__(kStreamBlock) void iota_kernel(uint32_t* __restrict
 // What bounds the ranges is a workgroup's pass over its chunk (L1 and the instructions per id), so their time follows
 // ratings / chunks: 100M ratings take 0.46 ms in 3 ranges, 0.81 in 7 (1.63 without the next tile's loads in flight), 1.55 in 15,
 // 2.95 from 17 to 32, up to a fifth more under Zipf(1.2).  A workgroup with ids of both sides makes two passes and the others wait
-// for it: 50M ratings of 1M + 200k ids took 1.67 ms in 15 ranges with one such and take 0.81 in 16 without.  In front of that come
-// 13 to 20 us: 160 KB of counters cleared, the sample, the counters' way to memory.
+// for it: 50M ratings of 1M + 200k ids took 1.67 ms in 15 ranges with one such and take 0.81 in 16 without.  (Calls repeated on the same
+// ratings; the one call of a training run on 100M ratings, 7 ranges, takes 1.1 ms under the profiler.)  In front of that come 13 to
+// 20 us: 160 KB of counters cleared, the sample, the counters' way to memory.
 // The tables' time follows the ids that find no slot.  50M ratings of 1M + 625k ids (21 ranges), hashed / ranges: flat 3.69 / 1.54 ms,
 // Zipf(0.8) 3.10 / 1.54, Zipf(1.0) 1.79 / 1.53, Zipf(1.1) 1.12 / 1.54, Zipf(1.2) 0.68 / 1.54.  The sample tells them apart: 7942, 6980,
 // 4653, 3441 and 2341 different hash values of both sides, and the line is at kHistDistinct.  With few ratings the tables are the
