@@ -85,6 +85,20 @@ __device__ __forceinline__ void process_full_chunk(Rule& rule, const Rating& my,
     typename Rule::Row ring[S];
     typename Rule::Info inf[S];
     static_for<0, S>([&](auto D) { inf[decltype(D)::value] = rule.no_row(); });
+    // Ratings that share a row with one of the A ratings before them, a bit each: the comparisons with the older slots
+    // (two per slot) are made once for the 64 ratings and the pipeline tests one bit instead of 18 of the 85 instructions
+    // that a rating of fp32 SGD took at k = 64 (a worker alone on its SIMD issues one every four clocks); leaving the
+    // comparisons out altogether was worth 0.3 to 0.8 ms of 4.4 to 5.8 ms per epoch of 8M ratings.
+    uint64_t shares = 0;
+    {
+        uint32_t ru = my.ru, rv = my.rv;
+        bool same = false;
+        static_for<0, A>([&](auto) {
+            ru = lane_below(ru); rv = lane_below(rv);
+            same |= ru == my.ru || rv == my.rv;
+        });
+        shares = __builtin_amdgcn_ballot_w64(same);
+    }
     auto fetch_rows = [&](auto SL, int j) {
         constexpr int sl = decltype(SL)::value;
         inf[sl] = rule.info(my, prep, j);
@@ -94,11 +108,13 @@ __device__ __forceinline__ void process_full_chunk(Rule& rule, const Rating& my,
     auto step = [&](auto D, int j) {
         constexpr int d = decltype(D)::value;
         row_arrived<CLS>(rule, ring[d], inf[d], 0);
-        static_for<0, A>([&](auto H) {
-            constexpr int h = A - decltype(H)::value;          // A, A-1, ..., 1: newest wins
-            constexpr int sh = (d - h + 2 * S) % S;
-            rule.forward(ring[d], inf[d], ring[sh], inf[sh]);
-        });
+        if (__builtin_expect((shares >> d) & 1ull, 0)) {
+            static_for<0, A>([&](auto H) {
+                constexpr int h = A - decltype(H)::value;          // A, A-1, ..., 1: newest wins
+                constexpr int sh = (d - h + 2 * S) % S;
+                rule.forward(ring[d], inf[d], ring[sh], inf[sh]);
+            });
+        }
         rule.template update<CLS, HOT, SCALED>(ring[d], inf[d], processed + (uint32_t)j);
     };
     static_for<0, A>([&](auto D) { fetch_rows(D, decltype(D)::value); });
@@ -108,6 +124,7 @@ __device__ __forceinline__ void process_full_chunk(Rule& rule, const Rating& my,
             fetch_rows(std::integral_constant<int, (d + A) % S>(), j0 + d + A);
             step(D, j0 + d);
         });
+        shares >>= S;
     }
     static_for<0, S>([&](auto D) {
         constexpr int d = decltype(D)::value;

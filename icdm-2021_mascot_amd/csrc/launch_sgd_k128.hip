@@ -1,4 +1,4 @@
-// fp32 SGD at k = 128, compiled with uniform branches structurised (build.py says why).
+// fp32 SGD at k = 128, a file of its own so that the launchers compile in parallel.
 #include "hogwild_launch.h"
 #include "rules_fp32.h"
 

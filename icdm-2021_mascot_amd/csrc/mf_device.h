@@ -44,6 +44,12 @@ template <int N, class T> __device__ __forceinline__ T row_ror(T x)
     return from_bits<T>((uint32_t)__builtin_amdgcn_mov_dpp((int)bits(x), 0x120 + N, 0xf, 0xf, true));
 }
 
+// Value held by the lane below (lane 0: all ones).
+__device__ __forceinline__ uint32_t lane_below(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)x, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
+}
+
 // Reduction steps: every lane ends with op(own, partner); op must be commutative.
 struct OpAdd { template <class T> __device__ __forceinline__ T operator()(T a, T b) const { return a + b; } };
 
@@ -129,39 +135,12 @@ __device__ __forceinline__ void row_add(half2_t* p, half2_t d)
     (void)__builtin_amdgcn_global_atomic_fadd_v2f16(global_ptr(p), d);
 }
 
-// A row seen through a buffer resource of `bytes` bytes: accesses past the end are dropped by the hardware,
-// so a window of 0 bytes turns a store into a no-op without a branch.  The fp32 rules' kernels with hot-row
-// code store rows this way: the store of a rating that is thinned, or whose change is added instead, is still
-// issued (and dropped), every rating then issues the same number of memory instructions on the straight path
-// and the compiler's counted waits (s_waitcnt vmcnt(N)) keep the look-ahead of the row loads.
+// A row seen through a buffer resource of `bytes` bytes: accesses past the end are dropped by the hardware, loads come
+// back zero (MASCOT's loads of rows of either precision).
 typedef __amdgpu_buffer_rsrc_t row_window_t;
 __device__ __forceinline__ row_window_t row_window(uint64_t row, uint32_t bytes)
 {
     return __builtin_amdgcn_make_buffer_rsrc((void*)row, 0, (int)bytes, 0x00020000 /* 32-bit data format, raw addressing */);
-}
-// COH: the sc1 cache policy of row_store's agent-scope stores
-template <bool COH> __device__ __forceinline__ void window_store(row_window_t w, uint32_t byte_offset, uint32_t v)
-{
-    __builtin_amdgcn_raw_buffer_store_b32(v, w, (int)byte_offset, 0, COH ? 16 : 0);
-}
-template <bool COH> __device__ __forceinline__ void window_store(row_window_t w, uint32_t byte_offset, uint16_t v)
-{
-    __builtin_amdgcn_raw_buffer_store_b16(v, w, (int)byte_offset, 0, COH ? 16 : 0);
-}
-template <bool COH> __device__ __forceinline__ void window_store(row_window_t w, uint32_t byte_offset, uint64_t v)
-{
-    typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2_t, v), w, (int)byte_offset, 0, COH ? 16 : 0);
-}
-
-// Adds through a row window (row_add's instructions in their buffer form: dropped when the window is closed).
-__device__ __forceinline__ void window_add(row_window_t w, uint32_t byte_offset, float d)
-{
-    (void)__builtin_amdgcn_raw_ptr_buffer_atomic_fadd_f32(d, w, (int)byte_offset, 0, 0);
-}
-__device__ __forceinline__ void window_add(row_window_t w, uint32_t byte_offset, half2_t d)
-{
-    (void)__builtin_amdgcn_raw_ptr_buffer_atomic_fadd_v2f16(d, w, (int)byte_offset, 0, 0);
 }
 
 // ---- counter-based generator -----------------------------------------------------------
@@ -244,6 +223,7 @@ __device__ __forceinline__ uint32_t xcd_id()
 // thin: bit0/bit1 skip the P/Q update, bit2/bit3 the P/Q row is a hot row (updates are added), bit4/bit5 the P/Q row is
 // a replicated row (the update goes to this XCD's copy: an ordinary cached store, or an add when bit2/bit3 is set as
 // well).  ru, rv: the row to address -- u, v themselves, or kReplicaRow | index of the replica row.
+constexpr uint32_t kHotBits = 0x3cu;          // Rating::thin: one of the two rows is a hot or a replicated row (a skipped update's row is hot)
 struct Rating { float r; uint32_t u; uint32_t v; uint32_t thin; uint32_t ru; uint32_t rv; };
 __device__ __forceinline__ Rating load_rating(const mf_node* R, uint32_t idx)
 {

@@ -458,13 +458,20 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
             const HV ruv = splat(r_h - dot);
             const HV gp = ruv * Q - lam_h * P;
             const HV gq = ruv * P - lam_h * Q;
-            if (!skip_p) {
+            if (CLS != 0 && HOT && __builtin_expect((i.thin & kHotBits) == 0u, 1)) {      // two ordinary rows, the most frequent kind: one branch
                 row.p[0] = bits(HV(__builtin_elementwise_fma(lr_p, gp, P)));
-                write_side_half<(CLS == 2 ? 1 : CLS), HOT>(row.p, lr_p * gp, i.pptr, i.thin);
-            }
-            if (!skip_q) {
                 row.q[0] = bits(HV(__builtin_elementwise_fma(lr_q, gq, Q)));
-                write_side_half<(CLS == 2 ? 1 : CLS), HOT>(row.q, lr_q * gq, i.qptr, i.thin >> 1);
+                store_side(row.p, i.pptr, false, lane);
+                store_side(row.q, i.qptr, false, lane);
+            } else {
+                if (!skip_p) {
+                    row.p[0] = bits(HV(__builtin_elementwise_fma(lr_p, gp, P)));
+                    write_side_half<(CLS == 2 ? 1 : CLS), HOT>(row.p, lr_p * gp, i.pptr, i.thin);
+                }
+                if (!skip_q) {
+                    row.q[0] = bits(HV(__builtin_elementwise_fma(lr_q, gq, Q)));
+                    write_side_half<(CLS == 2 ? 1 : CLS), HOT>(row.q, lr_q * gq, i.qptr, i.thin >> 1);
+                }
             }
             if (sampled) {
                 float g[E];

@@ -426,7 +426,7 @@ template <int K, bool COH> struct MuppetRule : DenseBase<K, COH> {
             row.p[e] = Base::template skips<CLS>(i.thin, 1u) ? row.p[e] : row.p[e] + dp[e];
             row.q[e] = Base::template skips<CLS>(i.thin, 2u) ? row.q[e] : row.q[e] + dq[e];
         }
-        this->template store<HOT>(row, i, dp, dq);
+        this->template store<CLS, HOT>(row, i, dp, dq);
         if (fwd != 32 && bwd != 32 && processed >= first_sample) {
             float gp[E], gq[E], sp2[E], sq2[E];
 #pragma unroll
@@ -652,7 +652,7 @@ template <int K, bool COH> struct AfpRule : DenseBase<K, COH> {
             row.p[e] = Base::template skips<CLS>(i.thin, 1u) ? row.p[e] : row.p[e] + dp[e];
             row.q[e] = Base::template skips<CLS>(i.thin, 2u) ? row.q[e] : row.q[e] + dq[e];
         }
-        this->template store<HOT>(row, i, dp, dq);
+        this->template store<CLS, HOT>(row, i, dp, dq);
         cur_iter += 1;
     }
     __device__ __forceinline__ void finish(const Params&, uint32_t) const {}

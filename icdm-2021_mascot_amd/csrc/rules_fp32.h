@@ -15,16 +15,10 @@ template <int K> struct DenseRow {
     static constexpr int E = K / 64;
     float p[E], q[E];
 };
-// What the dense fp32 rules broadcast per rating: the two rows as addresses (the matrix row, or this XCD's copy of a
-// replicated row) and Rating::thin with four more bits, one per store window of the hot-row code (DenseBase::store).
-// Addresses and window bits are computed once per chunk across the 64 lanes (DenseBase::prepare); per rating that costs
-// two more v_readlane where the scalar unit would otherwise rebuild both addresses from the row ids for the loads and
-// again for the stores and derive the four window sizes from thin (about forty scalar instructions per rating).
-// Measured at 100M ratings: 7 to 11 % per epoch at k = 64, where these rules are bound by instruction issue, nothing at
-// k = 128, where they are bound by the memory side; at 8M and 20M ratings, where a worker's chain of ratings is bound by
-// latency, 5 and 13 % at k = 128 and 20 % at k = 64.
+// What the dense rules broadcast per rating: the two rows as addresses (the matrix row, or this XCD's copy of a replicated
+// row), computed once per chunk across the 64 lanes (DenseBase::prepare), and Rating::thin.
 struct DenseAddrInfo { float r; uint32_t thin; uint64_t u, v; };
-struct DenseAddrPrep { uint64_t pu, pv; uint32_t thin; };
+struct DenseAddrPrep { uint64_t pu, pv; };
 
 template <int K, bool COH> struct DenseBase {
     static constexpr int E = K / 64;
@@ -48,29 +42,14 @@ template <int K, bool COH> struct DenseBase {
     __device__ __forceinline__ float step_of(float lrate, uint32_t thin, uint32_t bit) const { return (thin & bit) ? lrate_rep : lrate; }
     __device__ __forceinline__ float scale_of(uint32_t thin, uint32_t bit) const { return (thin & bit) ? rep_scale : 1.0f; }
 
-    // Bits of Info::thin above Rating::thin's six: the size of a row in bytes, a single bit, shifted left by 0..3 says
-    // that the user / item row's window for device-coherent stores and the user / item row's window for cached stores
-    // (the copy of a replicated row) is open, so that a window's size is one shift and one mask.
-    static constexpr uint32_t kRowBytes = K * 4u;
-    static_assert((kRowBytes & (kRowBytes - 1u)) == 0u && kRowBytes > 63u, "the window bits lie above Rating::thin's");
     // first element of a row of the matrix or, for a replicated row, of this XCD's copy
     template <class T> static __device__ __forceinline__ T* row_of(T* matrix, T* replicas, uint32_t row)
     {
         return ((row & kReplicaRow) ? replicas : matrix) + (size_t)(row & ~kReplicaRow) * K;
     }
-    // side 0: the user row, 1: the item row.  A row's new value is stored unless the update is thinned or added
-    // instead; a replicated row's copy is stored with an ordinary cached store (it stays in this XCD's L2) through a
-    // second window with that cache policy.
-    static __device__ __forceinline__ bool stores_row(uint32_t thin, int side) { return !((thin & (5u << side)) || (COH && (thin & (16u << side)))); }
-    static __device__ __forceinline__ bool stores_copy(uint32_t thin, int side) { return COH && (thin & (20u << side)) == (16u << side); }
     __device__ __forceinline__ Prep prepare(const Rating& my, bool) const
     {
-        Prep pr;
-        pr.pu = reinterpret_cast<uint64_t>(row_of(P, RP, my.ru));
-        pr.pv = reinterpret_cast<uint64_t>(row_of(Q, RQ, my.rv));
-        pr.thin = my.thin | (stores_row(my.thin, 0) ? kRowBytes : 0u) | (stores_row(my.thin, 1) ? kRowBytes << 1 : 0u)
-                  | (stores_copy(my.thin, 0) ? kRowBytes << 2 : 0u) | (stores_copy(my.thin, 1) ? kRowBytes << 3 : 0u);
-        return pr;
+        return Prep{reinterpret_cast<uint64_t>(row_of(P, RP, my.ru)), reinterpret_cast<uint64_t>(row_of(Q, RQ, my.rv))};
     }
     __device__ __forceinline__ int classify(const Rating& my, const Prep&, bool valid) const
     {
@@ -84,7 +63,7 @@ template <int K, bool COH> struct DenseBase {
     {
         Info i;
         i.r = bcast(my.r, j);
-        i.thin = bcast(pr.thin, j);
+        i.thin = bcast(my.thin, j);
         i.u = bcast(pr.pu, j);
         i.v = bcast(pr.pv, j);
         return i;
@@ -96,44 +75,40 @@ template <int K, bool COH> struct DenseBase {
 #pragma unroll
         for (int e = 0; e < E; ++e) { row.p[e] = row_load(pp + 64 * e); row.q[e] = row_load(qq + 64 * e); }
     }
-    // dp, dq: the change of each element (new - old as the rule computes it), added to a hot row.  Kernels with
-    // the hot-row code store through a row window (mf_device.h): one store per element and side is always
-    // issued, and dropped when the update is thinned or added instead.  (Measured at 100M ratings, k = 128: 3 % faster
-    // for these rules, whose epoch is bound by bytes in flight; the binary16 rules are bound by instruction issue,
-    // lose more to the dropped stores than the longer look-ahead gives them, and keep their branches.)
-    template <bool HOT> __device__ __forceinline__ void store(const Row& row, const Info& i, const float* dp, const float* dq) const
+    // One side of a rating that touches a hot row.  bits: the side's bits of Rating::thin, those of the user row.
+    template <int CLS> __device__ __forceinline__ void store_side(const float* row, const float* change, uint64_t at, uint32_t bits_) const
     {
-        float* pp = reinterpret_cast<float*>(i.u) + lane;
-        float* qq = reinterpret_cast<float*>(i.v) + lane;
-        if constexpr (!HOT) {
+        float* x = reinterpret_cast<float*>(at) + lane;
+        if ((bits_ & 20u) == 16u) {                  // this XCD's copy: an ordinary cached store
+#pragma unroll
+            for (int e = 0; e < E; ++e) row_store<false>(x + 64 * e, row[e]);
+        } else if (bits_ & 4u) {
+            if (CLS == 0 && (bits_ & 1u)) return;
+#pragma unroll
+            for (int e = 0; e < E; ++e) row_add(x + 64 * e, change[e]);
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e) row_store<COH>(x + 64 * e, row[e]);
+        }
+    }
+    // dp, dq: the change of each element (new - old as the rule computes it), added to a hot row.
+    // One test finds the rating whose two rows are both ordinary (a third to two thirds of them); the others branch three
+    // ways per side.  Every way issues E memory instructions per side, so the counted waits for the row loads in flight hold
+    // on all of them.  Bound by a worker's chain of instructions up to about 95M ratings, where stores to four row
+    // windows (ordinary and copy, each side, closed by a size of 0: some 25 scalar instructions and 2 E dropped stores per
+    // rating) cost more than the branches; with the shared-row bits of process_full_chunk, ms per epoch before -> now:
+    // fp32 SGD 8M ratings k = 64 4.43 -> 4.02, k = 128 5.77 -> 4.73, 100M 12.48 -> 11.9 and 20.4 -> 19.7; MPT 20M k = 128
+    // 6.96 -> 5.99; MuPPET k = 64 8M 10.31 -> 9.29, 100M 16.77 -> 15.97; AFP k = 128 9.67 -> 8.74 and 21.8 -> 21.3.
+    template <int CLS, bool HOT> __device__ __forceinline__ void store(const Row& row, const Info& i, const float* dp, const float* dq) const
+    {
+        if (HOT && __builtin_expect((i.thin & kHotBits) != 0u, 0)) {
+            store_side<CLS>(row.p, dp, i.u, i.thin);
+            store_side<CLS>(row.q, dq, i.v, i.thin >> 1);
+        } else {
+            float* pp = reinterpret_cast<float*>(i.u) + lane;
+            float* qq = reinterpret_cast<float*>(i.v) + lane;
 #pragma unroll
             for (int e = 0; e < E; ++e) { row_store<COH>(pp + 64 * e, row.p[e]); row_store<COH>(qq + 64 * e, row.q[e]); }
-        } else {
-            const bool add_p = (i.thin & 5u) == 4u, add_q = (i.thin & 10u) == 8u;
-            const row_window_t wp = row_window(i.u, i.thin & kRowBytes);
-            const row_window_t wq = row_window(i.v, (i.thin >> 1) & kRowBytes);
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                window_store<COH>(wp, (uint32_t)(lane + 64 * e) * 4u, bits(row.p[e]));
-                window_store<COH>(wq, (uint32_t)(lane + 64 * e) * 4u, bits(row.q[e]));
-            }
-            if constexpr (COH) {
-                const row_window_t rp = row_window(i.u, (i.thin >> 2) & kRowBytes);
-                const row_window_t rq = row_window(i.v, (i.thin >> 3) & kRowBytes);
-#pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    window_store<false>(rp, (uint32_t)(lane + 64 * e) * 4u, bits(row.p[e]));
-                    window_store<false>(rq, (uint32_t)(lane + 64 * e) * 4u, bits(row.q[e]));
-                }
-            }
-            if (add_p) {
-#pragma unroll
-                for (int e = 0; e < E; ++e) row_add(pp + 64 * e, dp[e]);
-            }
-            if (add_q) {
-#pragma unroll
-                for (int e = 0; e < E; ++e) row_add(qq + 64 * e, dq[e]);
-            }
         }
     }
     __device__ __forceinline__ void forward(Row& nxt, const Info& in, const Row& cur, const Info& ic) const
@@ -195,7 +170,7 @@ template <int K, bool COH> struct SgdRule : DenseBase<K, COH> {
             row.p[e] = Base::template skips<CLS>(i.thin, 1u) ? pe : pe + dp[e];
             row.q[e] = Base::template skips<CLS>(i.thin, 2u) ? qe : qe + dq[e];
         }
-        this->template store<HOT>(row, i, dp, dq);
+        this->template store<CLS, HOT>(row, i, dp, dq);
     }
     __device__ __forceinline__ void finish(const Params&, uint32_t) const {}
 };
@@ -239,7 +214,7 @@ template <int K, bool COH> struct MptRule : DenseBase<K, COH> {
             row.p[e] = Base::template skips<CLS>(i.thin, 1u) ? row.p[e] : row.p[e] + dp[e];
             row.q[e] = Base::template skips<CLS>(i.thin, 2u) ? row.q[e] : row.q[e] + dq[e];
         }
-        this->template store<HOT>(row, i, dp, dq);
+        this->template store<CLS, HOT>(row, i, dp, dq);
     }
     __device__ __forceinline__ void finish(const Params&, uint32_t) const {}
 };
@@ -373,6 +348,12 @@ template <int K, bool COH> struct MemQuantRule {
             nq[e] = qf[e] + dq[e];
         }
         // the register copy is what the row holds afterwards: the sum rounded to binary16
+        if (HOT && __builtin_expect((i.thin & kHotBits) == 0u, 1)) {
+            row.p = narrow(np); row.q = narrow(nq);
+            write_side(reinterpret_cast<uint16_t*>(i.u), row.p, dp, false, false);
+            write_side(reinterpret_cast<uint16_t*>(i.v), row.q, dq, false, false);
+            return;
+        }
         if (!(CLS == 0 && (i.thin & 1u))) { row.p = narrow(np); write_side(reinterpret_cast<uint16_t*>(i.u), row.p, dp, i.thin & 4u, i.thin & 16u); }
         if (!(CLS == 0 && (i.thin & 2u))) { row.q = narrow(nq); write_side(reinterpret_cast<uint16_t*>(i.v), row.q, dq, i.thin & 8u, i.thin & 32u); }
     }

@@ -613,6 +613,48 @@ def test_chunks_with_skipped_updates_take_the_general_loop_to_the_same_rows(k, v
 
 
 @pytest.mark.parametrize("k", [64, 128])
+@pytest.mark.parametrize("variant", ["single", "mpt", "muppet", "afp", "mem_quant"])
+def test_dense_rules_share_rows_at_every_distance_with_and_without_row_classes(k, variant):
+    """Ratings that share a row with one of the ratings whose rows are still in registers are found once per chunk, and a
+    rating with two ordinary rows is stored on a path of its own.  Workers with 9 users and 7 items of their own, so that
+    rows are shared at every distance on one side, the other or both, next to ratings that share none; ordinary and
+    replicated rows mixed at random must give the rows of the run without row classes, bit for bit: a replicated row
+    changes in one XCD's copy only and the merge returns that copy."""
+    import torch
+    h = mfutil.hip()
+    W, uc, window = 7, 3, 128
+    R, starts, P0, Q0 = mfutil.conflict_free_problem(900 + k, k, W, uc, window, users_per_worker=9, items_per_worker=7)
+    dt = np.float32
+    if variant == "mem_quant":
+        P0, Q0, dt = P0.astype(np.float16), Q0.astype(np.float16), np.float16
+    rng = np.random.default_rng(31 + k)
+    classes = [rng.choice([255, 253], size=m.shape[0]).astype(np.uint8) for m in (P0, Q0)]
+
+    def run(opt):
+        dR, dS, dP, dQ = to_dev(R), to_dev(starts), to_dev(P0), to_dev(Q0)
+        head = (dR.data_ptr(), R.size, dP.data_ptr(), dQ.data_ptr(), k, W, uc, window)
+        tail = (5, 0, dS.data_ptr(), mfutil.stream_ptr(), opt.ptr if opt else None)
+        if variant == "single":
+            h.mf_single_sgd_hogwild_opt(*head, LR, LAM, *tail)
+        elif variant == "mpt":
+            h.mf_mpt_sgd_hogwild_opt(*head, LR, 0x5240, 1000.0, *tail)          # binary16 50 = lambda x 1000
+        elif variant == "muppet":
+            sm, sn = torch.zeros(k, dtype=torch.float32, device="cuda"), torch.zeros(W, dtype=torch.float32, device="cuda")
+            h.mf_muppet_sgd_hogwild_opt(*head, LR, LAM, uc * window, sm.data_ptr(), sn.data_ptr(), 8, 8, *tail)
+        elif variant == "afp":
+            h.mf_afp_sgd_hogwild_opt(*head, LR, LAM, 1, *tail)
+        else:
+            h.mf_mem_quant_sgd_hogwild_opt(*head, LR, LAM, *tail)
+        torch.cuda.synchronize()
+        return from_dev(dP, dt, P0.shape), from_dev(dQ, dt, Q0.shape)
+
+    P1, Q1 = run(None)
+    P2, Q2 = run(mfutil.HogwildOptions(k, *classes))
+    assert np.any(P1 != P0) and np.any(Q1 != Q0)
+    assert np.array_equal(P2.view(np.uint8), P1.view(np.uint8)) and np.array_equal(Q2.view(np.uint8), Q1.view(np.uint8))
+
+
+@pytest.mark.parametrize("k", [64, 128])
 @pytest.mark.parametrize("variant", ["single", "mpt", "mascot", "muppet", "afp"])
 def test_hot_row_updates_add_up(orc, k, variant):
     """k wavefronts in k/4 workgroups update one hot item row at the same time.  User u's row is 0.5 * e_u, the item
