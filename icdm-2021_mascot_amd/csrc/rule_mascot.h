@@ -11,7 +11,7 @@
 // binary16 dot is bit-identical to the reference's sequence of roundings.
 //
 // The group search of the reference (two 32-wide register compares plus a shared-memory fallback per
-// rating, mascot_sgd_kernel.h:104-180) is replaced by one binary search per lane over the end-index
+// rating, mascot_sgd_kernel.h:104-180) is replaced by one search per lane over the end-index
 // table in LDS, done once for the 64 ratings of a chunk; the result is the row address, which is
 // what the per-rating loop broadcasts.
 #pragma once
@@ -124,25 +124,42 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
         __syncthreads();
     }
 
-    // min{g : idx <= end[g]}; rows of a group are idx - end[g-1] - 1 (mascot_sgd_kernel.h:104-143).
-    static __device__ __forceinline__ uint32_t search(const uint32_t* end, uint32_t groups, uint32_t idx)
+    // min{g : idx <= end[g]}, the last group if there is none, for both sides at once; rows of a group are
+    // idx - end[g-1] - 1 (mascot_sgd_kernel.h:104-143).  The result is first .. first + left, and a round asks three
+    // elements that cut the range in four (past the last but one: that one, and min() takes first back); `left` shrinks
+    // alike on all lanes.  What this costs is the latency of dependent LDS reads, once per chunk: two bisections one after
+    // the other (14 of them for 100 groups a side) took 3280 clocks of a chunk's 35,000 where a worker is alone on its
+    // SIMD; 100 groups take four rounds of six independent reads.
+    static __device__ __forceinline__ void search(const uint32_t* uend, const uint32_t* iend, uint32_t ug_n, uint32_t ig_n, uint32_t u, uint32_t v, uint32_t& ug, uint32_t& ig)
     {
-        uint32_t lo = 0, hi = groups - 1;
-        while (lo < hi) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (idx <= end[mid]) hi = mid; else lo = mid + 1;
+        const uint32_t last_u = ug_n > 1 ? ug_n - 2 : 0u, last_i = ig_n > 1 ? ig_n - 2 : 0u;
+        uint32_t left_u = ug_n - 1, left_i = ig_n - 1, first_u = 0, first_i = 0;
+        while (left_u | left_i) {
+            const uint32_t qu = left_u > 4u ? (left_u + 3u) >> 2 : 1u, qi = left_i > 4u ? (left_i + 3u) >> 2 : 1u;
+            uint32_t eu[3], ei[3];
+#pragma unroll
+            for (uint32_t t = 0; t < 3; ++t) {
+                const uint32_t au = first_u + (t + 1) * qu - 1, ai = first_i + (t + 1) * qi - 1;
+                eu[t] = uend[au < last_u ? au : last_u]; ei[t] = iend[ai < last_i ? ai : last_i];
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < 3; ++t) { first_u += eu[t] < u ? qu : 0u; first_i += ei[t] < v ? qi : 0u; }
+            left_u = left_u > 3u * qu && left_u - 3u * qu > qu - 1u ? left_u - 3u * qu : qu - 1u;
+            left_i = left_i > 3u * qi && left_i - 3u * qi > qi - 1u ? left_i - 3u * qi : qi - 1u;
         }
-        return lo;
+        ug = first_u < ug_n - 1 ? first_u : ug_n - 1;
+        ig = first_i < ig_n - 1 ? first_i : ig_n - 1;
     }
     __device__ __forceinline__ Prep prepare(const Rating& my, bool valid) const
     {
         Prep pr; pr.pptr = 0; pr.qptr = 0; pr.flags = kSkip;
         if (valid) {
-            const uint32_t ug = search(uend_s, user_groups, my.u);
-            const uint32_t ig = search(iend_s, item_groups, my.v);
-            const bool ok = my.u <= uend_s[ug] && my.v <= iend_s[ig];
-            const uint32_t urow = ug ? my.u - uend_s[ug - 1] - 1 : my.u;
-            const uint32_t irow = ig ? my.v - iend_s[ig - 1] - 1 : my.v;
+            uint32_t ug, ig;
+            search(uend_s, iend_s, user_groups, item_groups, my.u, my.v, ug, ig);
+            const uint32_t u_end = uend_s[ug], i_end = iend_s[ig], u_before = uend_s[ug ? ug - 1 : 0u], i_before = iend_s[ig ? ig - 1 : 0u];
+            const bool ok = (my.u <= u_end) & (my.v <= i_end);
+            const uint32_t urow = ug ? my.u - u_before - 1 : my.u;
+            const uint32_t irow = ig ? my.v - i_before - 1 : my.v;
             const uint32_t up = uprec_s[ug] ? 1u : 0u, ip = iprec_s[ig] ? 1u : 0u;
             // a rating that is skipped carries null pointers: forward() then matches it with no row
             pr.pptr = ok ? pptr_s[ug] + (uint64_t)urow * (K * (up ? 4u : 2u)) : 0ull;

@@ -344,6 +344,13 @@ def test_mascot_group_table_sizes(orc, k):
     _mascot_case(orc, k, 100, 1, 64, 400, 350, "mixed", first_sample=10, seed=63)
 
 
+@pytest.mark.parametrize("ug,ig", [(2, 3), (4, 5), (6, 16), (17, 18), (64, 65), (99, 100)])
+def test_mascot_group_search_asks_four_ways_on_both_sides(orc, ug, ig):
+    """Table sizes around the rounds of the search, different ones per side, so that one side's rounds end before the
+    other's: every rating must find its rows, bit for bit against the checker."""
+    _mascot_case(orc, 64, 40, 2, 128, ug, ig, "mixed", first_sample=2 * 128, seed=70 + ug)
+
+
 @pytest.mark.parametrize("k", [64, 128])
 def test_single_update_mascot_four_cases(orc, k):
     for up in (0, 1):
