@@ -76,8 +76,9 @@ template <class Rule> struct ahead_of<Rule, 2, std::void_t<decltype(Rule::kAhead
 template <int CLS, class Rule, class Row, class Info> __device__ __forceinline__ auto row_arrived(const Rule& rule, Row& row, const Info& i, int) -> decltype(rule.template arrive<CLS>(row, i), void()) { rule.template arrive<CLS>(row, i); }
 template <int CLS, class Rule, class Row, class Info> __device__ __forceinline__ void row_arrived(const Rule&, Row&, const Info&, long) {}
 
-template <class Rule, int CLS, bool HOT, bool SCALED>
-__device__ __forceinline__ void process_full_chunk(Rule& rule, const Rating& my, const typename Rule::Prep& prep, uint32_t processed)
+// before_last() is called before the last kRing ratings: loads for the next chunk that these ratings hide.
+template <class Rule, int CLS, bool HOT, bool SCALED, class BeforeLast>
+__device__ __forceinline__ void process_full_chunk(Rule& rule, const Rating& my, const typename Rule::Prep& prep, uint32_t processed, BeforeLast&& before_last)
 {
     constexpr int A = ahead_of<Rule, CLS>::value;
     constexpr int S = Rule::kRing;
@@ -126,6 +127,7 @@ __device__ __forceinline__ void process_full_chunk(Rule& rule, const Rating& my,
         });
         shares >>= S;
     }
+    before_last();
     static_for<0, S>([&](auto D) {
         constexpr int d = decltype(D)::value;
         if constexpr (d + A < S) fetch_rows(std::integral_constant<int, d + A>(), kWave - S + d + A);
@@ -184,30 +186,58 @@ void hogwild_kernel(Schedule s, typename Rule::Params prm)
             if (left > range_end - pp) left = range_end - pp;
             return left < (uint32_t)kWave ? (int)left : kWave;
         };
+        auto rating_index = [&](uint32_t st, uint32_t cc) -> uint32_t {
+            const uint32_t off = (cc + (uint32_t)lane) % s.nnz;
+            uint32_t idx = st + off;
+            if (idx >= s.nnz || idx < st) idx -= s.nnz;
+            return idx;
+        };
         auto fetch = [&](uint32_t st, uint32_t cc, int nn) -> Rating {
             Rating x = {0.f, 0u, 0u, 0u, 0u, 0u};
             if (lane < nn) {
-                uint32_t off = (cc + (uint32_t)lane) % s.nnz;
-                uint32_t idx = st + off;
-                if (idx >= s.nnz || idx < st) idx -= s.nnz;
-                x = load_rating(s.R, idx);
-                if constexpr (HOT) {
-                    const uint32_t rnd = (uint32_t)(mix64(s.epoch_key ^ (((uint64_t)idx << 20) ^ (uint64_t)wid ^ 0x7468696eull)) >> 40);
-                    const uint32_t ku = s.keep_u[x.u], kv = s.keep_v[x.v];
-                    // two independent draws, uniform over 0..254
-                    if (ku == kKeepReplicated || ku == kKeepReplicatedAdded) {
-                        x.thin |= ku == kKeepReplicated ? 16u : 20u; x.ru = kReplicaRow | (xcd * s.slots_u + s.slot_u[x.u]);
-                    } else if (ku != 255u) x.thin |= (((rnd & 0xfffu) * 255u) >> 12) > ku ? 5u : 4u;
-                    if (kv == kKeepReplicated || kv == kKeepReplicatedAdded) {
-                        x.thin |= kv == kKeepReplicated ? 32u : 40u; x.rv = kReplicaRow | (xcd * s.slots_v + s.slot_v[x.v]);
-                    } else if (kv != 255u) x.thin |= (((rnd >> 12) * 255u) >> 12) > kv ? 10u : 8u;
-                }
+                x = load_rating(s.R, rating_index(st, cc));
             }
             return x;
+        };
+        // What the hot-row tables say about a chunk's ratings, in two steps, because the second gather depends on the first:
+        // look_up requests the keep bytes (row 0's for lanes without a rating), mark gathers the slots of replicated rows.
+        // A chunk's ratings are requested when the chunk before it starts.  Rows of up to 256 bytes: its keep bytes before
+        // that chunk's last ratings, its slots when they are needed, so that of the three dependent latencies (3000 to 4500
+        // clocks of a chunk's 35,000 where a worker is alone on its SIMD) one is waited for.  Wider rows: all at once, as soon
+        // as the ratings are there.  ms per epoch, all at once -> in steps, runs of one side within 0.4 %: fp32 SGD k = 64
+        // 400k 3.81 -> 3.73, 8M 4.06 -> 4.00; MASCOT k = 128 8M 4.36 -> 4.29, k = 64 20M with some groups binary32 5.95 -> 5.85;
+        // -v 7 k = 64 8M 4.82 -> 4.69; MuPPET k = 64 100M 16.0 -> 15.9; but fp32 SGD k = 128 20M 5.68 -> 5.81, 100M 19.7 -> 19.9,
+        // MASCOT k = 128 100M with some groups binary32 14.75 -> 14.89.
+        constexpr bool kInSteps = Rule::kMaxRowBytes <= 256;
+        uint32_t keep_u = 255u, keep_v = 255u;
+        auto look_up = [&](const Rating& x) {
+            if constexpr (HOT) { keep_u = s.keep_u[x.u]; keep_v = s.keep_v[x.v]; }
+        };
+        auto mark = [&](Rating& x, uint32_t st, uint32_t cc, int nn) {
+            x.thin = 0u; x.ru = x.u; x.rv = x.v;
+            if constexpr (HOT) {
+                const uint32_t ku = lane < nn ? keep_u : 255u, kv = lane < nn ? keep_v : 255u;
+                const bool rep_u = ku == kKeepReplicated || ku == kKeepReplicatedAdded, rep_v = kv == kKeepReplicated || kv == kKeepReplicatedAdded;
+                uint32_t slot_u = 0u, slot_v = 0u;
+                if (rep_u) slot_u = s.slot_u[x.u];
+                if (rep_v) slot_v = s.slot_v[x.v];
+                if (ku < 255u && !rep_u) x.thin |= 4u;
+                if (kv < 255u && !rep_v) x.thin |= 8u;
+                if (__builtin_amdgcn_ballot_w64(ku <= kKeepThinnedMax || kv <= kKeepThinnedMax) != 0ull) {
+                    // two independent draws, uniform over 0..254; a row of keep value 254 is never skipped
+                    const uint32_t rnd = (uint32_t)(mix64(s.epoch_key ^ (((uint64_t)rating_index(st, cc) << 20) ^ (uint64_t)wid ^ 0x7468696eull)) >> 40);
+                    if ((x.thin & 4u) && (((rnd & 0xfffu) * 255u) >> 12) > ku) x.thin |= 1u;
+                    if ((x.thin & 8u) && (((rnd >> 12) * 255u) >> 12) > kv) x.thin |= 2u;
+                }
+                if (rep_u) { x.thin |= ku == kKeepReplicated ? 16u : 20u; x.ru = kReplicaRow | (xcd * s.slots_u + slot_u); }
+                if (rep_v) { x.thin |= kv == kKeepReplicated ? 32u : 40u; x.rv = kReplicaRow | (xcd * s.slots_v + slot_v); }
+            }
         };
         uint32_t start = window_of(ite);
         int n = chunk_len(c, processed);
         Rating my = fetch(start, c, n);
+        look_up(my);
+        mark(my, start, c, n);
         while (true) {
             // position of the chunk after this one, and its ratings, requested now
             uint32_t nprocessed = processed + (uint32_t)n;
@@ -219,30 +249,36 @@ void hogwild_kernel(Schedule s, typename Rule::Params prm)
                 if (nc >= s.update_vector_size) { nc = 0; ++nite; nstart = window_of(nite); }
                 nn = chunk_len(nc, nprocessed);
                 nmy = fetch(nstart, nc, nn);
+                if constexpr (!kInSteps) { look_up(nmy); mark(nmy, nstart, nc, nn); }
             }
             const bool valid = lane < n;
             typename Rule::Prep prep = rule.prepare(my, valid);
             const int cls = rule.classify(my, prep, valid);
             // classes (see the rules): 1 and 2 promise ratings that all take the same memory instructions; full
             // chunks of those run the straight-line pipeline, everything else the general one
+            auto next_keep = [&]() { if constexpr (kInSteps) look_up(nmy); };
             auto run = [&](auto Scaled) {
                 constexpr bool SC = decltype(Scaled)::value;
                 if (Rule::kClasses > 1 && cls == 1) {
-                    if (n == kWave) process_full_chunk<Rule, 1, HOT, SC>(rule, my, prep, processed);
-                    else process_chunk<Rule, 1, HOT, SC>(rule, my, prep, n, processed);
+                    if (n == kWave) { process_full_chunk<Rule, 1, HOT, SC>(rule, my, prep, processed, next_keep); return; }
+                    process_chunk<Rule, 1, HOT, SC>(rule, my, prep, n, processed);
                 } else if (Rule::kClasses > 2 && cls == 2 && n == kWave) {
-                    process_full_chunk<Rule, 2, HOT, SC>(rule, my, prep, processed);
+                    process_full_chunk<Rule, 2, HOT, SC>(rule, my, prep, processed, next_keep);
+                    return;
                 } else if (Rule::kClasses == 1 && n == kWave) {
-                    process_full_chunk<Rule, 0, HOT, SC>(rule, my, prep, processed);
+                    process_full_chunk<Rule, 0, HOT, SC>(rule, my, prep, processed, next_keep);
+                    return;
                 } else {
                     process_chunk<Rule, 0, HOT, SC>(rule, my, prep, n, processed);
                 }
+                next_keep();
             };
             // the few launches with longer steps on replicated rows (the first epoch by default) take their own copy of
             // the loops, so that every other launch pays nothing for them
             if (HOT && prm.rep_scale != 1.0f) run(std::true_type()); else run(std::false_type());
             if (!more) break;
             processed = nprocessed; c = nc; ite = nite; start = nstart; n = nn; my = nmy;
+            if constexpr (kInSteps) mark(my, start, c, n);
         }
     }
     rule.finish(prm, first_wid);                         // may synchronise the workgroup

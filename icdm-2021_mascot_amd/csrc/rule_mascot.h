@@ -35,8 +35,7 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
     // arithmetic and stores written for that case, each way issuing one store per side; 0 = anything, including ratings
     // that are skipped (an index outside the tables)
     static constexpr int kClasses = MIXED ? 3 : 2;
-    // no register limit is asked for: the build for all-binary16 runs fits six wavefronts per SIMD by itself (80), the
-    // build with the mixed path takes 83 (five), and held to 80 it spills and gains nothing (measured)
+    // no register limit is asked for: both builds fit six wavefronts per SIMD by themselves (76 and 80 registers)
     static constexpr int kMinWavesPerSimd = 1;
     using HV = typename std::conditional<E == 2, half2_t, half_t>::type;
 
@@ -54,6 +53,7 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
     };
     static constexpr uint32_t kReplicaSlotBytes = K * 4u;
     static constexpr int kK = K;
+    static constexpr int kMaxRowBytes = MIXED ? K * 4 : K * 2;      // of the chunks that are not the exception
     static void row_storage(const Params& a, RowStorage& u, RowStorage& v)
     {
         u.group_ptr = a.p; u.group_end = a.user_end; u.group_prec = a.user_prec; u.groups = a.user_groups;

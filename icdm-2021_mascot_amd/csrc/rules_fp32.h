@@ -29,6 +29,7 @@ template <int K, bool COH> struct DenseBase {
     // default run): its loop carries no selects for it; 0 = the general loop.
     static constexpr int kClasses = 2;
     static constexpr int kK = K;
+    static constexpr int kMaxRowBytes = K * 4;
     template <class Params> static void row_storage(const Params& a, RowStorage& u, RowStorage& v) { u.dense = a.p; v.dense = a.q; }
     float* P;
     float* Q;
@@ -247,6 +248,7 @@ template <int K, bool COH> struct MemQuantRule {
         return (row & kReplicaRow) ? replicas + (size_t)(row & ~kReplicaRow) * (2 * K) : matrix + (size_t)row * K;
     }
     static constexpr int kK = K;
+    static constexpr int kMaxRowBytes = K * 2;
     static void row_storage(const Params& a, RowStorage& u, RowStorage& v) { u.dense = a.p; u.elem_bytes = 2; v.dense = a.q; v.elem_bytes = 2; }
     __device__ __forceinline__ Prep prepare(const Rating& my, bool) const
     {
