@@ -89,6 +89,20 @@ struct Range {
 template <class P> static auto set_lds_stats(P& p, bool v) -> decltype(p.lds_stats, void()) { p.lds_stats = v; }
 static void set_lds_stats(...) {}
 
+// LDS that an ordinary launch of one build asks for: what the rule uses and, where the rule holds its hot-row build to
+// `held` workgroups per compute unit, enough that one workgroup more does not fit in the 160 KB (between a 1/(held + 1)th
+// and a 1/held-th of them, so that the allocation's granularity decides nothing).  Builds without the hot-row code launch with
+// their own LDS only: their registers let more workgroups in, and no table says how many there are.
+template <class Rule, bool HOT> constexpr size_t launch_lds(size_t own)
+{
+    constexpr int held = HOT ? hot_workgroups<Rule>::value : 0;
+    if constexpr (held > 0) {
+        constexpr size_t hold = (((160u << 10) / (held + 1)) & ~(size_t)1023) + 2048;
+        static_assert(held * hold <= (160u << 10) && (held + 1) * hold > (160u << 10), "no LDS size keeps exactly this many");
+        return own < hold ? hold : own;
+    }
+    return own;
+}
 template <class Rule, bool HOT>
 static int launch_hot(const char* who, const Call& c, const typename Rule::Params& prm0, size_t lds, void* stream, Range r);
 // Workgroups of `kernel` (kBlock threads, `lds` bytes of LDS of their own) that share a compute unit, and the LDS size
@@ -181,6 +195,7 @@ static int launch_hot(const char* who, const Call& c, const typename Rule::Param
     if (splits > windows) splits = windows ? windows : 1;
     bool first = true;
     scaled_steps(grid_for(s.num_workers));
+    lds = launch_lds<Rule, HOT>(lds);
     if (const size_t padded = lds_for_resident_cap(reinterpret_cast<const void*>(&hogwild_kernel<Rule, HOT>), lds, c.resident_workers, s.num_workers)) lds = padded;
     for (uint32_t i = 0; i < splits; ++i) {
         const uint32_t b = i == 0 ? r.begin : (first_window + (uint32_t)((uint64_t)windows * i / splits)) * s0.update_vector_size;
@@ -216,6 +231,7 @@ static float inflight_of(uint32_t num_workers, size_t lds, uint32_t resident_cap
 {
     int blocks = 0, dev = 0, cus = 0;
     const void* kernel = reinterpret_cast<const void*>(&hogwild_kernel<Rule, true>);
+    lds = launch_lds<Rule, true>(lds);
     // a launch held to resident_cap workers runs with the LDS size that does the holding
     if (const size_t padded = lds_for_resident_cap(kernel, lds, resident_cap, num_workers)) lds = padded;
     hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, kBlock, lds);

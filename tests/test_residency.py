@@ -1,0 +1,92 @@
+"""Workgroups per compute unit that the launches of the update kernels keep resident.  They are the updates in flight of a
+run whose workers fill the chip, so the hot-row tables, the first epoch's cap and every measured test RMSE go with them: a
+compiler that finds a few registers more or less must not change them unseen.  Read from the compiled kernels' registers and
+from what the launcher asks for."""
+import importlib
+import os
+import re
+import struct
+import subprocess
+
+import msgpack
+import pytest
+
+build = importlib.import_module("icdm-2021_mascot_amd.build")
+
+LDS = 160 << 10
+# (rule, k, coherent stores): workgroups per compute unit of launches without hot-row tables, with them, and the number the
+# rule holds the latter to (0: the registers say how many)
+RESIDENT = {
+    ("SgdRule", 128, True): (7, 6, 6), ("SgdRule", 128, False): (7, 6, 6),
+    ("SgdRule", 64, True): (7, 7, 0), ("SgdRule", 64, False): (7, 7, 0),
+    ("MascotPlainRule", 128, True): (7, 5, 5), ("MascotPlainRule", 128, False): (7, 5, 5),
+    ("MascotPlainRule", 64, True): (7, 7, 0), ("MascotPlainRule", 64, False): (7, 7, 0),
+    ("MascotBinary16Rule", 128, True): (7, 6, 0), ("MascotBinary16Rule", 128, False): (7, 6, 0),
+    ("MascotBinary16Rule", 64, True): (7, 7, 0), ("MascotBinary16Rule", 64, False): (7, 7, 0),
+    ("MascotRule", 128, True): (5, 4, 0), ("MascotRule", 128, False): (5, 4, 0),
+    ("MascotRule", 64, True): (6, 6, 0), ("MascotRule", 64, False): (6, 6, 0),
+}
+TEMPLATE = {"MascotPlainRule": "MascotRuleTILi%dELb%dELb0ELb1E", "MascotBinary16Rule": "MascotRuleTILi%dELb%dELb0ELb0E", "MascotRule": "MascotRuleTILi%dELb%dELb1ELb1E"}
+
+
+def _code_objects(path):
+    """The device code objects in a library's offload bundles."""
+    data = open(path, "rb").read()
+    for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data):
+        entries, = struct.unpack_from("<Q", data, m.end())
+        at = m.end() + 8
+        for _ in range(entries):
+            offset, size, length = struct.unpack_from("<QQQ", data, at)
+            if build.ARCH.encode() in data[at + 24:at + 24 + length]:
+                yield data[m.start() + offset:m.start() + offset + size]
+            at += 24 + length
+
+
+def _kernels(elf):
+    """The kernel records of one code object's metadata note."""
+    sections, = struct.unpack_from("<Q", elf, 0x28)
+    entry, count = struct.unpack_from("<HH", elf, 0x3a)
+    for i in range(count):
+        kind, _, _, offset, _ = struct.unpack_from("<IQQQQ", elf, sections + i * entry + 4)
+        if kind == 7:                                    # a note: name size, contents size, type, name, contents
+            name, size, _ = struct.unpack_from("<III", elf, offset)
+            at = offset + 12 + (name + 3) // 4 * 4
+            yield from msgpack.unpackb(elf[at:at + size])["amdhsa.kernels"]
+
+
+@pytest.fixture(scope="module")
+def by_registers():
+    """Mangled kernel name -> workgroups of four wavefronts, one per SIMD, that its registers let in: 512 vector registers
+    in eights and 800 scalar ones in sixteens per SIMD."""
+    if not os.path.exists(build.LIB):
+        build.build()
+    out = {}
+    for elf in _code_objects(build.LIB):
+        for k in (k for k in _kernels(elf) if "hogwild_kernel" in k[".name"]):
+            out[k[".name"]] = min(512 // (-(-k[".vgpr_count"] // 8) * 8), 800 // (-(-k[".sgpr_count"] // 16) * 16), 8)
+    return out
+
+
+@pytest.mark.parametrize("rule,k,coherent", sorted(RESIDENT))
+def test_registers_and_holds_give_the_residency_the_tables_are_built_for(by_registers, rule, k, coherent):
+    free, hot, held = RESIDENT[rule, k, coherent]
+    name = TEMPLATE.get(rule, rule + "ILi%dELb%dE") % (k, coherent)
+    got = [[w for n, w in by_registers.items() if re.search(r"hogwild_kernelINS_\d+" + name + "EELb%dE" % b, n)] for b in (0, 1)]
+    assert [len(g) for g in got] == [1, 1], "one kernel per build"
+    assert got[0][0] == free
+    assert min(got[1][0], held or 8) == hot
+
+
+def test_the_launcher_holds_hot_row_builds_only(tmp_path):
+    """launch_lds of every build, compiled for the host: the LDS asked for lets exactly the held number of workgroups in,
+    larger group tables are kept whole, and a launch without hot-row tables asks for nothing beyond its own."""
+    src = ['#include "hogwild_launch.h"', '#include "rule_mascot.h"', '#include "rules_fixed_point.h"', '#include "rules_fp32.h"', "using namespace mf;"]
+    for (rule, k, coherent), (_, _, held) in sorted(RESIDENT.items()):
+        r = "%s<%d, %s>" % (rule, k, "true" if coherent else "false")
+        src.append("static_assert(launch_lds<%s, false>(0) == 0 && launch_lds<%s, false>(4096) == 4096);" % (r, r))
+        lds = "launch_lds<%s, true>(4096)" % r
+        src.append("static_assert(%s * %d <= %d && %s * %d > %d && launch_lds<%s, true>(65536) == 65536);" % (lds, held, LDS, lds, held + 1, LDS, r) if held else
+                   "static_assert(%s == 4096);" % lds)
+    path = tmp_path / "launch_lds_check.hip"
+    path.write_text("\n".join(src) + "\n")
+    subprocess.run([build.HIPCC, "--offload-arch=" + build.ARCH, "-std=c++17", "--cuda-host-only", "-fsyntax-only", "-Wno-unused-function", "-I" + build.CSRC, str(path)], check=True)
