@@ -252,6 +252,11 @@ template <int K, bool COH> struct MuppetRule : DenseBase<K, COH> {
         void* rep_p; void* rep_q; float rep_scale;
     };
     static constexpr bool kSplittable = false;     // per-worker statistics span the whole launch
+    // k = 128: the hot-row build's 71 registers would let seven workgroups in.  Two fifths more updates in flight, and half as
+    // many again in the first epoch, in which too long a step makes this rule run away at random (HotRows::install): they were
+    // measured with five, and with six where rows are stored through the caches.  An epoch of 100M ratings takes 22.3 ms with
+    // seven, 23.0 with five.
+    static constexpr int kHotWorkgroups = K == 128 ? (COH ? 5 : 6) : 0;
     float lrate, lambda; uint32_t first_sample; float* sum_updated_val; int fwd, bwd;
     float sum_norms_reg;
     float grad_acc[K / 64];
@@ -486,7 +491,10 @@ template <int K, bool COH> struct AfpRule : DenseBase<K, COH> {
     static constexpr int E = Base::E;
     static constexpr int J = K / 32;
     static constexpr int kAhead = 1, kRing = 4;    // as for MuPPET: three ratings ahead measured no faster (k = 128) or slower (k = 64)
-    static constexpr int kMinWavesPerSimd = 6;     // 24 wavefronts per CU: 6144 workers resident at a time (85 VGPRs otherwise: 5 per SIMD, 5120)
+    static constexpr int kMinWavesPerSimd = 6;     // 24 wavefronts per CU: 6144 workers resident at a time
+    // k = 64: the hot-row build with coherent stores fits 64 registers, seven workgroups; a run's test RMSE was measured with the
+    // six of before (an epoch of 100M ratings takes 12.8 ms with seven, 12.9 with six).
+    static constexpr int kHotWorkgroups = K == 64 && COH ? 6 : 0;
     static constexpr bool kSplittable = false;    // the per-worker quantiser state lives for one launch
     struct Params { float* p; float* q; float lrate; float lambda; int afp_epoch; int init_threshold; bool accumulate; void* rep_p; void* rep_q; float rep_scale; };
     float lrate, lambda; int afp_epoch, init_threshold;

@@ -187,6 +187,9 @@ template <int K, bool COH> struct MptRule : DenseBase<K, COH> {
     static constexpr int E = Base::E;
     static constexpr int kAhead = 3, kRing = 8;
     static constexpr bool kSplittable = true;
+    // k = 128: the hot-row build's 73 registers would let a sixth workgroup in, and with it a fifth more updates in flight
+    // (an epoch of 100M ratings 19.8 -> 19.7 ms) than a run's test RMSE and its first epoch, two workgroups, were measured with.
+    static constexpr int kHotWorkgroups = K == 128 ? 5 : 0;
     struct Params { float* p; float* q; float lrate; uint16_t scaled_lambda_half; float scaling_factor; bool accumulate; void* rep_p; void* rep_q; float rep_scale; };
     float lrate, scaling_factor_rev;
     half_t lambda_h, scaling_factor_h;

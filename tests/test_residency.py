@@ -1,7 +1,7 @@
 """Workgroups per compute unit that the launches of the update kernels keep resident.  They are the updates in flight of a
 run whose workers fill the chip, so the hot-row tables, the first epoch's cap and every measured test RMSE go with them: a
 compiler that finds a few registers more or less must not change them unseen.  Read from the compiled kernels' registers and
-from what the launcher asks for."""
+from what the launcher asks for, and on the GPU from the number of updates in flight that the library reports."""
 import importlib
 import os
 import re
@@ -11,6 +11,8 @@ import subprocess
 import msgpack
 import pytest
 
+import mfutil
+
 build = importlib.import_module("icdm-2021_mascot_amd.build")
 
 LDS = 160 << 10
@@ -19,6 +21,14 @@ LDS = 160 << 10
 RESIDENT = {
     ("SgdRule", 128, True): (7, 6, 6), ("SgdRule", 128, False): (7, 6, 6),
     ("SgdRule", 64, True): (7, 7, 0), ("SgdRule", 64, False): (7, 7, 0),
+    ("MptRule", 128, True): (7, 5, 5), ("MptRule", 128, False): (7, 5, 5),
+    ("MptRule", 64, True): (7, 7, 0), ("MptRule", 64, False): (7, 7, 0),
+    ("MuppetRule", 128, True): (7, 5, 5), ("MuppetRule", 128, False): (7, 6, 6),
+    ("MuppetRule", 64, True): (7, 7, 0), ("MuppetRule", 64, False): (7, 7, 0),
+    ("AfpRule", 128, True): (6, 6, 0), ("AfpRule", 128, False): (6, 6, 0),
+    ("AfpRule", 64, True): (7, 6, 6), ("AfpRule", 64, False): (7, 7, 0),
+    ("MemQuantRule", 128, True): (7, 7, 0), ("MemQuantRule", 128, False): (7, 7, 0),
+    ("MemQuantRule", 64, True): (7, 7, 0), ("MemQuantRule", 64, False): (7, 7, 0),
     ("MascotPlainRule", 128, True): (7, 5, 5), ("MascotPlainRule", 128, False): (7, 5, 5),
     ("MascotPlainRule", 64, True): (7, 7, 0), ("MascotPlainRule", 64, False): (7, 7, 0),
     ("MascotBinary16Rule", 128, True): (7, 6, 0), ("MascotBinary16Rule", 128, False): (7, 6, 0),
@@ -90,3 +100,18 @@ def test_the_launcher_holds_hot_row_builds_only(tmp_path):
     path = tmp_path / "launch_lds_check.hip"
     path.write_text("\n".join(src) + "\n")
     subprocess.run([build.HIPCC, "--offload-arch=" + build.ARCH, "-std=c++17", "--cuda-host-only", "-fsyntax-only", "-Wno-unused-function", "-I" + build.CSRC, str(path)], check=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("k", [64, 128])
+@pytest.mark.parametrize("version,rule", [(5, "SgdRule"), (4, "MptRule"), (3, "MuppetRule"), (2, "AfpRule"), (7, "MemQuantRule"), (1, "MascotBinary16Rule")])
+def test_updates_in_flight_are_counted_with_that_residency(version, rule, k):
+    """A full chip, and the first epoch of a run on it: half the workers, in whole workgroups per compute unit."""
+    import torch
+    h = mfutil.hip()
+    hot = RESIDENT[rule, k, True][1]
+    workgroup = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    per_worker = h.lib.mf_hogwild_inflight(version, k, 1, 5, 5)
+    full = h.lib.mf_hogwild_inflight(version, k, 1000000, 5, 5) / per_worker
+    assert full == hot * workgroup
+    assert h.lib.mf_hogwild_inflight_capped(version, k, 1000000, 5, 5, int(full) // 2) / per_worker == hot // 2 * workgroup
