@@ -620,31 +620,34 @@ def test_chunks_with_skipped_updates_take_the_general_loop_to_the_same_rows(k, v
 
 
 @pytest.mark.parametrize("k", [64, 128])
+@pytest.mark.parametrize("W,uc,window", [(7, 3, 128), (9, 4, 70)])
 @pytest.mark.parametrize("variant", ["single", "mpt", "muppet", "afp", "mem_quant"])
-def test_dense_rules_share_rows_at_every_distance_with_and_without_row_classes(k, variant):
+def test_dense_rules_share_rows_at_every_distance_with_and_without_row_classes(orc, k, W, uc, window, variant):
     """Ratings that share a row with one of the ratings whose rows are still in registers are found once per chunk, and a
     rating with two ordinary rows is stored on a path of its own.  Workers with 9 users and 7 items of their own, so that
-    rows are shared at every distance on one side, the other or both, next to ratings that share none; ordinary and
-    replicated rows mixed at random must give the rows of the run without row classes, bit for bit: a replicated row
-    changes in one XCD's copy only and the merge returns that copy."""
+    rows are shared at every distance on one side, the other or both, next to ratings that share none, in chunks of 64 and
+    (windows of 70) of 6 whose successor is looked up behind the general loop.  Against the checker bit for bit: without row
+    classes; with ordinary rows and rows stored to one XCD's copy mixed at random (the merge returns the one copy that
+    changed); and with rows whose updates are added, in memory (254) and to a copy (252), among them."""
     import torch
     h = mfutil.hip()
-    W, uc, window = 7, 3, 128
     R, starts, P0, Q0 = mfutil.conflict_free_problem(900 + k, k, W, uc, window, users_per_worker=9, items_per_worker=7)
     dt = np.float32
     if variant == "mem_quant":
-        P0, Q0, dt = P0.astype(np.float16), Q0.astype(np.float16), np.float16
-    rng = np.random.default_rng(31 + k)
-    classes = [rng.choice([255, 253], size=m.shape[0]).astype(np.uint8) for m in (P0, Q0)]
+        P0, Q0, dt = orc.f2h(P0).reshape(P0.shape), orc.f2h(Q0).reshape(Q0.shape), np.uint16
+    elif variant == "mpt":
+        P0, Q0 = (orc.h2f(orc.f2h(m)).reshape(m.shape) for m in (P0, Q0))
+    lam_h = orc.lib.orc_float2half(np.float32(LAM) * np.float32(1000.0))
 
-    def run(opt):
+    def run(*keep):
+        opt = mfutil.HogwildOptions(k, *keep) if keep else None
         dR, dS, dP, dQ = to_dev(R), to_dev(starts), to_dev(P0), to_dev(Q0)
         head = (dR.data_ptr(), R.size, dP.data_ptr(), dQ.data_ptr(), k, W, uc, window)
         tail = (5, 0, dS.data_ptr(), mfutil.stream_ptr(), opt.ptr if opt else None)
         if variant == "single":
             h.mf_single_sgd_hogwild_opt(*head, LR, LAM, *tail)
         elif variant == "mpt":
-            h.mf_mpt_sgd_hogwild_opt(*head, LR, 0x5240, 1000.0, *tail)          # binary16 50 = lambda x 1000
+            h.mf_mpt_sgd_hogwild_opt(*head, LR, lam_h, 1000.0, *tail)
         elif variant == "muppet":
             sm, sn = torch.zeros(k, dtype=torch.float32, device="cuda"), torch.zeros(W, dtype=torch.float32, device="cuda")
             h.mf_muppet_sgd_hogwild_opt(*head, LR, LAM, uc * window, sm.data_ptr(), sn.data_ptr(), 8, 8, *tail)
@@ -655,10 +658,41 @@ def test_dense_rules_share_rows_at_every_distance_with_and_without_row_classes(k
         torch.cuda.synchronize()
         return from_dev(dP, dt, P0.shape), from_dev(dQ, dt, Q0.shape)
 
-    P1, Q1 = run(None)
-    P2, Q2 = run(mfutil.HogwildOptions(k, *classes))
-    assert np.any(P1 != P0) and np.any(Q1 != Q0)
-    assert np.array_equal(P2.view(np.uint8), P1.view(np.uint8)) and np.array_equal(Q2.view(np.uint8), Q1.view(np.uint8))
+    want = [P0.copy(), Q0.copy()]
+    head = (k, R.ctypes.data, R.size, want[0].ctypes.data, want[1].ctypes.data, W, uc, window, LR, LAM)
+    tail = (0, 0, starts.ctypes.data, 1)
+    if variant == "single":
+        orc.lib.orc_sgd_epoch(*head, *tail)
+    elif variant == "mpt":
+        orc.lib.orc_mpt_epoch(*head, 1000.0, *tail)
+    elif variant == "muppet":
+        sm, sn = np.zeros(k, np.float32), np.zeros(W, np.float32)
+        orc.lib.orc_muppet_epoch(*head, uc * window, sm.ctypes.data, sn.ctypes.data, 8, 8, *tail)
+    elif variant == "afp":
+        orc.lib.orc_afp_epoch(*head, 1, *tail)
+    else:
+        orc.lib.orc_mem_quant_epoch(*head, *tail)
+
+    def exact(got):
+        return all(np.array_equal(g.view(np.uint8), w.view(np.uint8)) for g, w in zip(got, want))
+
+    assert np.any(want[0] != P0) and np.any(want[1] != Q0)
+    assert exact(run())
+    rng = np.random.default_rng(31 + k)
+    stored, added = ([rng.choice(values, size=m.shape[0]).astype(np.uint8) for m in (P0, Q0)] for values in ([255, 253], [252, 253, 254, 255]))
+    assert exact(run(*stored))
+    got = run(*added)
+    if variant != "mem_quant":
+        assert exact(got)          # binary32: old + change is the stored value
+    else:
+        # binary16: each added change is rounded before the sum is, up to one ulp of the larger of change and result per update
+        # against the rounded sum, and what it moves in the rating's other row is less by lr * |row|^2, 0.01: twice one ulp of
+        # the row's largest element per update of the row
+        for g, w, old, ids in zip(got, want, (P0, Q0), (R["u"], R["i"])):
+            g, w, old = (orc.h2f(m).reshape(m.shape).astype(np.float64) for m in (g, w, old))
+            count = np.bincount(ids, minlength=w.shape[0])
+            ulp = np.spacing(np.maximum(np.abs(w), np.abs(old)).max(1).astype(np.float16)).astype(np.float64)
+            assert np.all(np.abs(g - w) <= (2 * count * ulp)[:, None])
 
 
 @pytest.mark.parametrize("k", [64, 128])
