@@ -41,10 +41,10 @@ DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-co
 #   MPT                    4.61 -> 4.59  12.06 -> 12.08       6.08 -> 6.05   20.15 -> 20.14
 #   AFP                    8.42 -> 8.37  13.45 -> 13.40       9.64 -> 9.65   21.72 -> 21.70
 #   MuPPET                10.22 -> 10.30 16.97 -> 16.82      11.34 -> 11.32  23.60 -> 23.53
-# MASCOT's mixed epochs of 250M ratings are level.  fp32 SGD at k = 128 lost 0.6 to 1 % while its hot-row build stored through
-# row windows; with the branches it has now it gains more than any (an epoch of 8M ratings 5.53 -> 4.73 ms, 100M 19.82 -> 19.72).
+# MASCOT's mixed epochs of 250M ratings are level.  The rows of fp32 SGD, MPT, AFP and MuPPET were taken while their hot-row builds
+# stored through row windows; with the branches they have now fp32 SGD at k = 128 gains too (8M 5.26 -> 4.47, 100M 19.90 -> 19.86).
 UNIFORM_BRANCH_FLAGS = ["-mllvm", "-structurizecfg-skip-uniform-regions=true", "-mllvm", "-enable-tail-merge=false"]
-STRUCTURISED = set()      # files compiled without these flags: none
+STRUCTURISED = set()      # files compiled without these flags (none at present; flags are recorded file by file for them)
 EXTRA_FLAGS = os.environ.get("MF_HIPCC_FLAGS", "").split()
 KERNEL_SOURCES = ["launch_mascot_plain.hip", "launch_mascot_sampled.hip", "launch_mascot_binary16.hip", "launch_muppet.hip", "launch_afp.hip", "hogwild_launch.hip", "launch_sgd_k128.hip",
                   "launch_mem_quant.hip", "aux_kernels.hip", "sort_shuffle.hip", "launch_mascot.hip"]

@@ -10,8 +10,9 @@
 //     rating j+kAhead are requested before rating j is reduced, updated and stored, so kAhead+1
 //     ratings of a wavefront are in flight and a row's latency hides behind kAhead updates;
 //   * a row requested early can be stale if one of the kAhead ratings in between updates the same
-//     row.  Row identities are wave-uniform scalars, so that is a scalar compare per older slot; on
-//     a match the freshly computed row is forwarded from that slot's registers.  A worker therefore
+//     row.  The ratings of a full chunk for which that is so are found once for the chunk, across the
+//     lanes, and only for those the row identities (wave-uniform scalars) are compared with the older
+//     slots' and the freshly computed row is forwarded from a slot's registers.  A worker therefore
 //     applies its own updates strictly in order (what a bit-exact check needs); different workers
 //     still race on P and Q without atomics -- that is Hogwild.
 #pragma once
@@ -213,7 +214,7 @@ void hogwild_kernel(Schedule s, typename Rule::Params prm)
         // clocks of a chunk's 35,000 where a worker is alone on its SIMD) one is waited for.  Wider rows: all at once, as soon
         // as the ratings are there.  ms per epoch, all at once -> in steps, runs of one side within 0.4 %: fp32 SGD k = 64
         // 400k 3.81 -> 3.73, 8M 4.06 -> 4.00; MASCOT k = 128 8M 4.36 -> 4.29, k = 64 20M with some groups binary32 5.95 -> 5.85;
-        // -v 7 k = 64 8M 4.82 -> 4.69; MuPPET k = 64 100M 16.0 -> 15.9; but fp32 SGD k = 128 20M 5.68 -> 5.81, 100M 19.7 -> 19.9,
+        // -v 7 k = 64 8M 4.82 -> 4.69; MuPPET k = 64 100M 16.0 -> 15.9; but fp32 SGD k = 128 20M 5.68 -> 5.81, 100M (then seven workgroups per compute unit) 19.7 -> 19.9,
         // MASCOT k = 128 100M with some groups binary32 14.75 -> 14.89.
         constexpr bool kInSteps = Rule::kMaxRowBytes <= 256;
         uint32_t keep_u = 255u, keep_v = 255u;

@@ -293,7 +293,8 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
             row.q[0] = (i.flags & 2u) ? row.q[0] : ((row.q[0] >> shift) & 0xffffu);
         }
     }
-    // selects, no branches: a branch here would sit between the row loads and their first use
+    // selects, no branches of its own: full chunks call this for ratings that share a row only, short ones for every rating,
+    // between the row loads and their first use
     __device__ __forceinline__ void forward(Row& nxt, const Info& in, const Row& cur, const Info& ic) const
     {
         // skipped ratings and empty slots have null pointers; copies between two of those are never used
@@ -411,10 +412,10 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
         }
     }
 
-    // Writes one side of an update: the new row `r` (raw registers) or, for an added row, its change `d` (binary32; a
+    // These write one side of an update: the new row `r` (raw registers) or, for an added row, its change `d` (binary32; a
     // binary16 row receives it rounded, which is exact when it was computed in binary16).  bits: the side's thin bits
     // shifted down -- 4 the row is added to, 16 the row is this XCD's copy of a replicated row.
-    // the same for a binary16 row whose change was computed in binary16 (mascot_sgd_kernel.h:188-278)
+    // A binary16 row whose change was computed in binary16 (mascot_sgd_kernel.h:188-278):
     template <int CLS, bool HOT> __device__ __forceinline__ void write_side_half(const uint32_t* r, HV d, uint64_t ptr, uint32_t bits_) const
     {
         if (HOT && (bits_ & 20u) == 16u) store_side<false>(r, ptr, false, lane);
@@ -478,7 +479,7 @@ template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
             const HV ruv = splat(r_h - dot);
             const HV gp = ruv * Q - lam_h * P;
             const HV gq = ruv * P - lam_h * Q;
-            if (CLS != 0 && HOT && __builtin_expect((i.thin & kHotBits) == 0u, 1)) {      // two ordinary rows, the most frequent kind: one branch
+            if (CLS != 0 && HOT && __builtin_expect((i.thin & kHotBits) == 0u, 1)) {      // two ordinary rows (a third of the ratings at 8M, a tenth at 100M): one branch
                 row.p[0] = bits(HV(__builtin_elementwise_fma(lr_p, gp, P)));
                 row.q[0] = bits(HV(__builtin_elementwise_fma(lr_q, gq, Q)));
                 store_side(row.p, i.pptr, false, lane);

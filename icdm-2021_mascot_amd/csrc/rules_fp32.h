@@ -93,12 +93,12 @@ template <int K, bool COH> struct DenseBase {
         }
     }
     // dp, dq: the change of each element (new - old as the rule computes it), added to a hot row.
-    // One test finds the rating whose two rows are both ordinary (a third to two thirds of them); the others branch three
-    // ways per side.  Every way issues E memory instructions per side, so the counted waits for the row loads in flight hold
-    // on all of them.  Bound by a worker's chain of instructions up to about 95M ratings, where stores to four row
+    // One test finds the rating whose two rows are both ordinary (with the tables of a run 43 % of them at 400k ratings, 34 %
+    // at 8M, 20 % at 20M, 10 to 14 % at 100M); the others branch three ways per side.  In chunks without skipped updates every
+    // way issues E memory instructions per side, so the counted waits for the row loads in flight hold on all of them.  Bound by a worker's chain of instructions up to about 95M ratings, where stores to four row
     // windows (ordinary and copy, each side, closed by a size of 0: some 25 scalar instructions and 2 E dropped stores per
     // rating) cost more than the branches; with the shared-row bits of process_full_chunk, ms per epoch before -> now:
-    // fp32 SGD 8M ratings k = 64 4.43 -> 4.02, k = 128 5.77 -> 4.73, 100M 12.48 -> 11.9 and 20.4 -> 19.7; MPT 20M k = 128
+    // fp32 SGD 8M ratings k = 64 4.43 -> 4.02, k = 128 5.77 -> 4.73, 100M 12.48 -> 11.9 and 20.3 -> 19.9; MPT 20M k = 128
     // 6.96 -> 5.99; MuPPET k = 64 8M 10.31 -> 9.29, 100M 16.77 -> 15.97; AFP k = 128 9.67 -> 8.74 and 21.8 -> 21.3.
     template <int CLS, bool HOT> __device__ __forceinline__ void store(const Row& row, const Info& i, const float* dp, const float* dq) const
     {
@@ -146,8 +146,9 @@ template <int K, bool COH> struct SgdRule : DenseBase<K, COH> {
     static constexpr int E = Base::E;
     static constexpr int kAhead = 3, kRing = 8;
     static constexpr bool kSplittable = true;
-    // k = 128: the hot-row build's 71 registers would let a seventh workgroup in, which leaves a sixth more updates in flight:
-    // single elements of an epoch of 100M ratings then lie 0.66 of the model's root mean square from where six leave them.
+    // k = 128: the hot-row build's 71 registers would let a seventh workgroup in.  An epoch of 100M ratings would take 19.4 ms
+    // instead of 19.9, with a sixth more updates in flight: single elements then lie 0.66 of the model's root mean square
+    // from where six leave them.
     static constexpr int kHotWorkgroups = K == 128 ? 6 : 0;
     struct Params { float* p; float* q; float lrate; float lambda; bool accumulate; void* rep_p; void* rep_q; float rep_scale; };
     float lrate, lambda;
