@@ -22,7 +22,7 @@ namespace mf {
 // SAMPLED = false compiles the sampled-statistics code out: the kernel for launches in which no rating is sampled.
 // MIXED = false compiles the straight-line path for chunks of mixed precisions out (such chunks take the general path,
 // so the results are the same): the kernel for runs in which every group is still binary16, which then keeps the
-// registers of the binary16 path alone and with them one more resident wavefront per SIMD.
+// registers of the binary16 path alone (76 instead of 80 at k = 128) and runs six workgroups per compute unit, not five.
 template <int K, bool COH, bool SAMPLED, bool MIXED = true> struct MascotRuleT {
     static constexpr int E = K / 64;                        // elements per lane
     static constexpr int kAhead = 3, kRing = 8;
