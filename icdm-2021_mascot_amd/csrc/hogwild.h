@@ -144,7 +144,7 @@ template <class Rule> struct min_waves_per_simd<Rule, std::void_t<decltype(Rule:
 
 // A rule may hold the launches of its hot-row build to a number of workgroups per compute unit (kHotWorkgroups; 0 = what
 // registers and LDS let in).  Workgroups per compute unit are updates in flight once the chip is full: the hot-row tables
-// are built for them, the first epoch runs at half of them and the test RMSE of a run was measured with them, so they must
+// are built for them, the first epoch is held to half of them and the test RMSE of a run was measured with them, so they must
 // not move when the compiler finds a few registers more or less.
 template <class Rule, class = void> struct hot_workgroups { static constexpr int value = 0; };
 template <class Rule> struct hot_workgroups<Rule, std::void_t<decltype(Rule::kHotWorkgroups)>> { static constexpr int value = Rule::kHotWorkgroups; };

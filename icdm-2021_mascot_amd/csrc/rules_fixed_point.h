@@ -252,9 +252,9 @@ template <int K, bool COH> struct MuppetRule : DenseBase<K, COH> {
         void* rep_p; void* rep_q; float rep_scale;
     };
     static constexpr bool kSplittable = false;     // per-worker statistics span the whole launch
-    // k = 128: the hot-row build's 71 registers would let seven workgroups in.  Two fifths more updates in flight, and half as
-    // many again in the first epoch, in which too long a step makes this rule run away at random (HotRows::install): they were
-    // measured with five, and with six where rows are stored through the caches.  An epoch of 100M ratings takes 22.3 ms with
+    // k = 128: the hot-row build's 71 registers would let seven workgroups in.  That is two fifths more updates in flight,
+    // and a first epoch, in which too long a step makes this rule run away at random (HotRows::install), with tables for half as many
+    // again: both were measured with five, and with six where rows are stored through the caches.  An epoch of 100M ratings takes 22.3 ms with
     // seven, 23.0 with five.
     static constexpr int kHotWorkgroups = K == 128 ? (COH ? 5 : 6) : 0;
     float lrate, lambda; uint32_t first_sample; float* sum_updated_val; int fwd, bwd;

@@ -300,7 +300,7 @@ struct HotRows {
             const double per_worker = mf_hogwild_inflight(prm.version, (int)prm.k, 1, user_groups, item_groups);
             const uint32_t resident = per_worker > 0 ? (uint32_t)(inflight / per_worker + 0.5) : 0;
             capped = (uint32_t)(resident * (double)prm.early_inflight);
-            // what a launch held to that many workers really keeps in flight (whole workgroups per compute unit)
+            // what the occupancy query counts for a launch held to that many workers (whole workgroups per compute unit)
             low_inflight = capped >= 1 ? mf_hogwild_inflight_capped(prm.version, (int)prm.k, prm.num_workers, user_groups, item_groups, capped) : 0.0;
             if (!(low_inflight > 0 && low_inflight < inflight)) low_inflight = 0;
         }

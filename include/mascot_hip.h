@@ -137,8 +137,9 @@ int mf_hot_row_table(const uint32_t* counts, uint32_t rows, uint32_t n, float in
  * min(num_workers, wavefronts the device keeps resident for that kernel) x the ratings a wavefront keeps in flight
  * (4; 2 for MuPPET and AFP).  Asks the HIP runtime for the kernel's occupancy on the current device. */
 float mf_hogwild_inflight(uint32_t version, int k, uint32_t num_workers, uint32_t user_groups, uint32_t item_groups);
-/* The same for launches with mf_hogwild_options::resident_workers set (0 = not set): what such a launch really keeps
- * in flight -- the cap works in whole workgroups per compute unit and does nothing to a launch that is below it anyway. */
+/* The same for launches with mf_hogwild_options::resident_workers set (0 = not set): the cap works in whole workgroups
+ * per compute unit and does nothing to a launch that is below it anyway.  The count is the occupancy query's; where the
+ * cap comes to three workgroups per compute unit the hardware, which hands LDS out in larger units, runs two. */
 float mf_hogwild_inflight_capped(uint32_t version, int k, uint32_t num_workers, uint32_t user_groups, uint32_t item_groups, uint32_t resident_workers);
 /* Seeded synthetic ratings (no counterpart in the reference, whose data sets are downloaded): users and items are
  * drawn independently from Zipf(alpha) over a random permutation of the ids; a rating is
